@@ -1,11 +1,14 @@
 // Stateless fp32-boundary operators: bf_cuda_gemm_f32 and bf_cuda_conv2d_f32
 // (drop-ins for reference src/cuda_ops.cu:147-208).
 //
-// Both run the bf16 MFMA GEMM core.  Operands arrive as fp32 and are rounded
-// to bf16 while they are staged into LDS; the convolution never materialises
-// an im2col matrix (conv_core.h gathers taps straight from NCHW).
+// Both multiply on the bf16 matrix cores.  Operands arrive as fp32 and are
+// rounded to bf16 while they are staged into LDS; the convolution never
+// materialises an im2col matrix (conv_direct.h reads every tap from one staged
+// patch; conv_core.h gathers taps straight from NCHW for the shapes that does
+// not take).
 #include "bf_cuda_ops.h"
 #include "conv_core.h"
+#include "conv_direct.h"
 
 #include <climits>
 
@@ -188,6 +191,112 @@ void conv_dispatch_tile(const ConvGeom &g, int Co, const float *x, const float *
     }
 }
 
+template <class T>
+void conv_direct_launch(const DirectConv &d, int batches, bool vec, bool flat, hipStream_t s) {
+    const dim3 grid(d.tiles_y * d.tiles_x * d.tiles_c * batches), block(T::kThreads);
+    if (d.up_h) {
+        if (vec && flat)
+            hipLaunchKernelGGL((conv_direct_kernel<T, true, true, true>), grid, block, 0, s, d);
+        else if (vec)
+            hipLaunchKernelGGL((conv_direct_kernel<T, true, true, false>), grid, block, 0, s, d);
+        else if constexpr (T::BC < 128)  // (the largest tile is not offered to scalar transposed layers)
+            hipLaunchKernelGGL((conv_direct_kernel<T, true, false, false>), grid, block, 0, s, d);
+    } else if (vec && flat) {
+        hipLaunchKernelGGL((conv_direct_kernel<T, false, true, true>), grid, block, 0, s, d);
+    } else if (vec) {
+        hipLaunchKernelGGL((conv_direct_kernel<T, false, true, false>), grid, block, 0, s, d);
+    } else {
+        hipLaunchKernelGGL((conv_direct_kernel<T, false, false, false>), grid, block, 0, s, d);
+    }
+}
+
+// Plans every tile and launches the one with the least estimate; false when
+// none takes the shape.
+bool conv_direct_best(const DirectConv &d, int batches, int kh, bool wv, bool flat, hipStream_t s) {
+    using Big = DirectTile<128, 160, 2, 2, 8, 9, 1>;
+    using Mid = DirectTile<64, 128, 2, 2, 4, 9, 1>;
+    using Low = DirectTile<32, 64, 1, 4, 4, 9, 1>;
+    using Min = DirectTile<32, 32, 2, 2, 4, 9, 1>;
+    struct Choice { DirectConv d; float us; int tile; bool vec; } best{d, -1.f, -1, false};
+    auto offer = [&](auto tile, int id, bool vec) {
+        Choice c{d, 0.f, id, vec};
+        const bool quads = vec && !d.up_h;
+        if (direct_plan<decltype(tile)>(c.d, batches, kh, quads, vec && flat, &c.us)) {
+            if (!vec) c.us *= 1.1f;  // four times the load instructions
+            if (best.tile < 0 || c.us < best.us) best = c;
+        }
+    };
+    for (bool vec : {true, false}) {
+        if (vec && !wv) continue;
+        if (vec || !d.up_h) offer(Big{}, 0, vec);
+        offer(Mid{}, 1, vec);
+        offer(Low{}, 2, vec);
+        offer(Min{}, 3, vec);
+    }
+    const bool f = best.vec && flat;
+    switch (best.tile) {
+        case 0: conv_direct_launch<Big>(best.d, batches, best.vec, f, s); break;
+        case 1: conv_direct_launch<Mid>(best.d, batches, best.vec, f, s); break;
+        case 2: conv_direct_launch<Low>(best.d, batches, best.vec, f, s); break;
+        case 3: conv_direct_launch<Min>(best.d, batches, best.vec, f, s); break;
+        default: return false;
+    }
+    return true;
+}
+
+// The direct kernel for this convolution, or false when the shape is not one
+// it takes: more than 36 taps, a transposed layer whose kernel is not its
+// stride (or padded, or cropped), an image or weight tensor of 1 GiB or more,
+// or a stride so large that no patch fits.
+//
+// Tiles, by least estimate (direct_estimate): 128 x 160 (eight loader waves)
+// for full grids, 64 x 128 and 32 x 64 below, 32 x 32 where the grid would
+// leave CUs idle.  Measured on MI355X against the im2col gather: 3x3 256 -> 256
+// on 6 x 32 x 88 433 -> 39 us (515 TFLOP/s), transposed 2x2 256 -> 256 on 90 x
+// 90 376 -> 37 us.  By tile: 3x3 512 -> 128 on 64 x 64 27 us with 32 x 64 tiles
+// (40 with 64 x 128, 30 with 32 x 32), 3x3 64 -> 64 on 2 x 128 x 128 12 us with
+// 64 x 128 (18 with 128 x 160, 19 with 32 x 64).
+bool conv_direct(const bf_cuda_conv2d_desc *c, const float *x, const float *w, const float *b,
+                 float *y, hipStream_t s) {
+    DirectConv d{};
+    d.x = x; d.w = w; d.bias = b; d.y = y;
+    d.Ci = c->input_channels; d.relu = c->relu;
+    d.IH = c->input_height; d.IW = c->input_width;
+    const long long hw = (long long)d.IH * d.IW, taps = (long long)c->kernel_height * c->kernel_width;
+    const long long columns = c->output_channels * (c->transpose ? taps : 1);
+    const long long x_bytes = 4 * hw * d.Ci, w_bytes = 4 * taps * d.Ci * c->output_channels;
+    if (taps > 36 || hw >= 1ll << 28 || x_bytes >= 1ll << 30 || w_bytes >= 1ll << 30) return false;
+    d.columns = (int)columns;
+    d.x_bytes = (uint32_t)x_bytes;
+    d.w_bytes = (uint32_t)w_bytes;
+    int kh = c->kernel_height;
+    if (c->transpose) {
+        if (c->kernel_height != c->stride_height || c->kernel_width != c->stride_width ||
+            c->padding_height || c->padding_width ||
+            c->output_height != (long long)d.IH * kh || c->output_width != (long long)d.IW * c->kernel_width)
+            return false;
+        d.up_h = kh; d.up_w = c->kernel_width; d.up_ow = d.IW;
+        d.pairs = kh == 2 && d.up_w == 2 && ((uintptr_t)y & 7) == 0;
+        d.khw = d.kw = kh = 1;
+        d.SH = d.SW = 1;
+    } else {
+        d.khw = (int)taps; d.kw = c->kernel_width;
+        d.SH = c->stride_height; d.SW = c->stride_width;
+        d.PH = c->padding_height; d.PW = c->padding_width;
+        d.OH = c->output_height; d.OW = c->output_width;
+    }
+    // One tap at stride one: the image is one row of pixels.
+    const bool one = c->transpose || (d.khw == 1 && d.SH == 1 && d.SW == 1 && !d.PH && !d.PW &&
+                                      d.OH == d.IH && d.OW == d.IW);
+    if (one) {
+        d.OH = d.IH = 1;
+        d.OW = d.IW = (int)hw;
+    }
+    const bool wv = aligned16(w) && (c->transpose ? d.columns % 4 == 0 : (long long)d.Ci * d.khw % 4 == 0);
+    const bool flat = wv && one && hw % 4 == 0 && aligned16(x);
+    return conv_direct_best(d, c->batches, kh, wv, flat, s);
+}
+
 }  // namespace
 
 extern "C" int bf_cuda_conv2d_f32(const bf_cuda_conv2d_desc *d, const float *input,
@@ -220,7 +329,9 @@ extern "C" int bf_cuda_conv2d_f32(const bf_cuda_conv2d_desc *d, const float *inp
     const long long tiles = ((long long)g.M + 127) / 128 * ((Co + 31LL) / 32);
     if (tiles > INT_MAX) return fail(error, cap, "HIP convolution grid is too large");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (Co <= 32)
+    if (conv_direct(d, input, weight, bias, output, s))
+        ;
+    else if (Co <= 32)
         conv_dispatch_tile<Tile<128, 32, 32, 4, 1>>(g, Co, input, weight, bias, output, d->relu, s);
     else if (Co <= 64)
         conv_dispatch_tile<Tile<128, 64, 32, 4, 1>>(g, Co, input, weight, bias, output, d->relu, s);

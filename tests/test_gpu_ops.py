@@ -219,3 +219,66 @@ def test_gemm_panel_equals_tiled_core(device, case):
     if special:
         assert np.array_equal(np.isnan(a), np.isnan(want)) and np.array_equal(np.isinf(a), np.isinf(want))
     _tight(a, want, f"panel gemm {case}")
+
+
+# Fields as CONV_CASES.  Shapes at the edges of the direct kernel's tiles and
+# channel blocks: one channel; blocks of 32 with one channel over, one under
+# and seven short; whole and ragged output-channel tiles (33, 129); kernels
+# taller than wide; 36 taps (the most it takes) and 49 (the gather core's);
+# padding wider than the kernel's reach; a stride that leaves one pixel per
+# patch row; an output larger and one smaller than the input defines; more
+# than one column tile and image; a flat 1x1 with an odd pixel count;
+# transposed 2x2 on odd widths, 3x3 and 1x3 kernels, and a padded one (the
+# gather core's).
+DIRECT_CASES = {
+    "one_channel": (2, 1, 33, 9, 11, 3, 3, 1, 1, 1, 1, 9, 11, 0, 1),
+    "tail_33": (1, 33, 40, 12, 20, 3, 3, 1, 1, 1, 1, 12, 20, 0, 0),
+    "tail_31_vec": (1, 60, 129, 17, 23, 3, 3, 1, 1, 1, 1, 17, 23, 0, 1),
+    "tail_25": (3, 25, 64, 7, 50, 3, 3, 2, 2, 1, 1, 4, 25, 0, 0),
+    "tall": (1, 12, 20, 15, 14, 5, 2, 1, 2, 2, 0, 15, 7, 0, 0),
+    "taps_36": (1, 9, 17, 14, 13, 6, 6, 1, 1, 2, 3, 13, 14, 0, 0),
+    "taps_49": (1, 9, 17, 14, 13, 7, 7, 1, 1, 3, 3, 14, 13, 0, 0),
+    "wide_pad": (1, 8, 16, 6, 5, 3, 3, 1, 1, 4, 5, 12, 13, 0, 0),
+    "stride_7": (1, 20, 24, 40, 50, 3, 3, 7, 9, 1, 1, 6, 6, 0, 1),
+    "larger_out": (1, 16, 16, 8, 8, 3, 3, 1, 1, 1, 1, 11, 10, 0, 0),
+    "smaller_out": (2, 16, 16, 9, 9, 3, 3, 1, 1, 1, 1, 5, 4, 0, 0),
+    "full_tiles": (2, 64, 256, 32, 88, 3, 3, 1, 1, 1, 1, 32, 88, 0, 1),
+    "flat_odd": (2, 70, 45, 9, 31, 1, 1, 1, 1, 0, 0, 9, 31, 0, 0),
+    "flat_vec": (2, 68, 130, 12, 30, 1, 1, 1, 1, 0, 0, 12, 30, 0, 1),
+    "strided_1x1": (1, 24, 40, 13, 18, 1, 1, 2, 3, 0, 0, 7, 6, 0, 0),
+    "up_2x2_odd": (2, 37, 19, 5, 7, 2, 2, 2, 2, 0, 0, 10, 14, 1, 1),
+    "up_2x2_vec": (1, 40, 66, 10, 12, 2, 2, 2, 2, 0, 0, 20, 24, 1, 0),
+    "up_3x3": (1, 10, 5, 6, 8, 3, 3, 3, 3, 0, 0, 18, 24, 1, 0),
+    "up_1x3": (1, 10, 8, 6, 8, 1, 3, 1, 3, 0, 0, 6, 24, 1, 0),
+    "up_padded": (1, 10, 8, 6, 8, 2, 2, 2, 2, 1, 1, 10, 14, 1, 0),
+}
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("case", sorted(DIRECT_CASES))
+def test_conv_direct_edges(device, case, special):
+    """Against the float64 sum over bf16-rounded operands (1e-5 of the RMS:
+    fp32 sums of at most 576 products), with and without Inf / NaN inputs,
+    which may reach only the sums they belong to."""
+    print(f"[case] conv {case} special={special}", flush=True)
+    d, x, w, b, got = run_conv(device, DIRECT_CASES[case], special)
+    want = convref.conv_abi(d, x, w, b, round_inputs=bf16_round)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    _tight(got, want, case)
+
+
+def test_conv_unaligned_operands(device):
+    """Input, weights and output off the 16-byte grid (scalar fetches, and
+    float stores in a transposed layer)."""
+    import bfhip
+    import torch
+    rng = np.random.default_rng(21)
+    for shape, wshape, kw in (((1, 32, 12, 16), (48, 32, 3, 3), dict(padding=(1, 1))),
+                              ((1, 32, 12, 16), (48, 32, 1, 1), {}),
+                              ((1, 32, 12, 16), (32, 24, 2, 2), dict(stride=(2, 2), transpose=True))):
+        x, w = _t(rng.standard_normal(shape), device), _t(rng.standard_normal(wshape) / 17, device)
+        want = bfhip.conv2d_f32(x, w, **kw)
+        off = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)  # noqa: E731
+        out = off(torch.zeros_like(want))
+        bfhip.conv2d_f32(off(x), off(w), out=out, **kw)
+        _tight(out.cpu().numpy(), want.cpu().numpy(), f"unaligned conv {wshape}")
