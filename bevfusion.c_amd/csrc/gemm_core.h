@@ -68,8 +68,11 @@ struct LoadRowsBf16 {
     }
 };
 
-// Row-major fp32 operand converted to bf16 on the way into LDS.  VEC requires
+// Row-major fp32 operand rounded to bf16 on the way into LDS.  VEC requires
 // K % 4 == 0, ld % 4 == 0 and a 16-byte aligned base; otherwise elementwise.
+// load() only issues the reads (an element past the rows or K reads the
+// operand's first element); store() masks, rounds and writes them, so they
+// stay in flight across the caller's MFMAs.
 template <int ROWS, int BK, int THREADS, bool VEC>
 struct LoadRowsF32 {
     static constexpr int kPerRow = BK / 8;
@@ -77,44 +80,42 @@ struct LoadRowsF32 {
     static constexpr int kPer = (kChunks + THREADS - 1) / THREADS;
     const float *base;
     int ld, rows, K;
-    int r0, tid;
-    bf16x8 st[kPer];
+    int r0, tid, k0;
+    float raw[kPer][8];
 
     __device__ void setup(int origin, int t) { r0 = origin; tid = t; }
-    __device__ void load(int k0) {
+    __device__ void load(int k) {
+        k0 = k;
 #pragma unroll
         for (int p = 0; p < kPer; ++p) {
             const int c = tid + p * THREADS;
             const int gr = r0 + c / kPerRow, gk = k0 + (c % kPerRow) * 8;
-            bf16x8 v = {};
-            if (c < kChunks && gr < rows) {
-                const float *src = base + (size_t)gr * ld + gk;
-                if (VEC) {
-                    if (gk < K) {  // K % 8 == 0 is not required: K % 4 == 0 is
-                        const float4 lo = *reinterpret_cast<const float4 *>(src);
-                        v[0] = to_bf16(lo.x); v[1] = to_bf16(lo.y);
-                        v[2] = to_bf16(lo.z); v[3] = to_bf16(lo.w);
-                        if (gk + 4 < K) {
-                            const float4 hi = *reinterpret_cast<const float4 *>(src + 4);
-                            v[4] = to_bf16(hi.x); v[5] = to_bf16(hi.y);
-                            v[6] = to_bf16(hi.z); v[7] = to_bf16(hi.w);
-                        }
-                    }
-                } else {
+            const bool row = c < kChunks && gr < rows;
+            const float *src = base + (row ? (size_t)gr * ld : 0);
+            if (VEC) {  // K % 8 == 0 is not required: K % 4 == 0 is
 #pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        if (gk + e < K) v[e] = to_bf16(src[e]);
+                for (int h = 0; h < 2; ++h) {
+                    const float4 f = *reinterpret_cast<const float4 *>(src + (gk + 4 * h < K ? gk + 4 * h : 0));
+                    raw[p][4 * h] = f.x; raw[p][4 * h + 1] = f.y;
+                    raw[p][4 * h + 2] = f.z; raw[p][4 * h + 3] = f.w;
                 }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) raw[p][e] = src[gk + e < K ? gk + e : 0];
             }
-            st[p] = v;
         }
     }
     __device__ void store(bf16 *lds) const {
 #pragma unroll
         for (int p = 0; p < kPer; ++p) {
             const int c = tid + p * THREADS;
+            const int gk = k0 + (c % kPerRow) * 8;
+            const int in = r0 + c / kPerRow < rows ? K - gk : 0;  // elements of the chunk that exist
+            bf16x8 v;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = to_bf16(e < in ? raw[p][e] : 0.0f);
             if (c < kChunks)
-                *reinterpret_cast<bf16x8 *>(lds + (c / kPerRow) * (BK + 8) + (c % kPerRow) * 8) = st[p];
+                *reinterpret_cast<bf16x8 *>(lds + (c / kPerRow) * (BK + 8) + (c % kPerRow) * 8) = v;
         }
     }
 };

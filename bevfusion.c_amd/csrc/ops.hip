@@ -42,7 +42,7 @@ void gemm_f32_launch(const float *x, const float *w, const float *b, float *y, i
 // (32-deep MFMA steps in increasing k) and the bias is added after it, so the
 // two paths agree bit for bit.  Requires K % 4 == 0, N % 4 == 0 and 16-byte
 // aligned X, W, bias and Y.  Measured on MI355X at config 1 (M = 11264,
-// K = 96, N = 288; HIP-graph replays): 8.05 us (the tiled core: 9.4 us).
+// K = 96, N = 288; HIP-graph replays): 8.05 us (the tiled core: 8.8 us).
 // Staging W per workgroup is what costs: with all 288 columns in one
 // workgroup and W converted through registers it took 6.3 of 12.5 us; half
 // the columns per workgroup and eight waves brought that form to 7.8 us,
@@ -51,6 +51,10 @@ constexpr int kPanelWaves = 8;
 constexpr int kPanelThreads = kPanelWaves * kWave;
 constexpr int kPanelRows = 16 * kPanelWaves;
 constexpr int kPanelMaxFrags = 9;  // column blocks per half: N <= 288
+// Below this the panels leave most CUs idle (K = 96, N = 288, panel against
+// tiled core: M = 500 6.1 vs 3.1 us, 3000 6.5 vs 4.6, 9000 8.2 vs 7.5, 11264
+// 8.4 vs 8.8).
+constexpr int kPanelMinRows = 10240;
 
 inline int panel_cols(int N) { return 16 * (((N + 15) / 16 + 1) / 2); }  // per column half
 inline size_t panel_lds_bytes(int N, int ks) { return (size_t)panel_cols(N) * 8 * ks * 16; }
@@ -137,7 +141,7 @@ __global__ __launch_bounds__(kPanelThreads) void gemm_f32_panel_kernel(
 // The panel kernel for (M, K, N), or false when the shape is not one it takes.
 bool gemm_f32_panel(const float *x, const float *w, const float *b, float *y, int M, int K, int N,
                     int relu, hipStream_t s) {
-    if (K > 128 || (K & 3) || (N & 3) || N <= 144 || N > 2 * 16 * kPanelMaxFrags ||
+    if (M < kPanelMinRows || K > 128 || (K & 3) || (N & 3) || N <= 144 || N > 2 * 16 * kPanelMaxFrags ||
         (long long)N * K * 4 >= (1ll << 31) || !aligned16(x) || !aligned16(w) || !aligned16(y) ||
         (b && !aligned16(b)))
         return false;
@@ -155,21 +159,155 @@ bool gemm_f32_panel(const float *x, const float *w, const float *b, float *y, in
     return true;
 }
 
+// Few or thin outputs: one wave per 16 x 16 output tile, no LDS staging.  The
+// lanes load their fp32 operand fragments (lane l: row l & 15, eight k at
+// 8 (l >> 4)) kAhead MFMA steps ahead and round them in registers; KW waves
+// of a workgroup take consecutive shares of the steps and their partial tiles
+// are added in LDS in wave order.  Bound by load latency: a step costs about
+// 0.8 us and KW of them run side by side, where the tiled core's k-loop takes
+// 1 us per 128 columns.  Every tile reads its own rows of both operands, so
+// this loses once the 16 x 16 tiles outnumber the CUs several times.  WM tiles
+// below one another share a workgroup when the reduction is short (KW = 1).
+// MI355X, eight waves against the best tiled core: 200 x 128 -> 256 2.8 vs 3.0
+// us, 1068 x 744 -> 41 4.6 vs 8.0, 7 x 1340 -> 2404 5.5 vs 12, 6 x 2386 -> 4 12
+// vs 72; four tiles, one wave each: 100000 x 8 -> 16 4.8 vs 8.1.
+template <int WM, int KW, bool VEC>
+__global__ __launch_bounds__(64 * WM * KW) void gemm_f32_thin_kernel(
+    const float *__restrict__ x, const float *__restrict__ w, const float *__restrict__ bias,
+    float *__restrict__ y, int M, int K, int N, int tiles_n, int relu) {
+    constexpr int kAhead = 4;
+    static_assert(WM == 1 || KW == 1, "one tile per workgroup when the waves split the reduction");
+    __shared__ f32x4 part[KW > 1 ? (KW - 1) * 64 : 1];
+    const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int kw = KW > 1 ? wave : 0, pid = xcd_swizzle((int)blockIdx.x, (int)gridDim.x);
+    const int m0 = 16 * (pid / tiles_n * WM + (KW > 1 ? 0 : wave)), n0 = pid % tiles_n * 16;
+    const int steps = (K + 31) / 32, per = (steps + KW - 1) / KW;
+    const int s0 = kw * per, s1 = min(steps, s0 + per);
+    const uint32_t row = (uint32_t)K * 4u, at = (uint32_t)(lane & 15) * row;
+    // Rows past M or N and columns past K read as zero.
+    const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x + (size_t)min(m0, M) * K, (uint32_t)max(0, min(16, M - m0)) * row);
+    const __amdgpu_buffer_rsrc_t wr = buffer_rsrc(w + (size_t)n0 * K, (uint32_t)min(16, N - n0) * row);
+
+    float xv[kAhead][8], wv[kAhead][8];
+    auto fetch = [&](__amdgpu_buffer_rsrc_t r, uint32_t k, float (&v)[8]) {
+        if constexpr (VEC) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const f32x4 f = buffer_f32x4(r, k + 4 * h < (uint32_t)K ? at + 4u * k + 16 * h : kDmaOutOfRange);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[4 * h + e] = f[e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = buffer_f32(r, k + e < (uint32_t)K ? at + 4u * (k + e) : kDmaOutOfRange);
+        }
+    };
+    auto load = [&](int p, int s) {
+        const uint32_t k = 32u * s + 8u * (lane >> 4);
+        fetch(xr, k, xv[p]);
+        fetch(wr, k, wv[p]);
+    };
+#pragma unroll
+    for (int p = 0; p < kAhead; ++p)
+        if (s0 + p < s1) load(p, s0 + p);
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int s = s0; s < s1; s += kAhead) {
+#pragma unroll
+        for (int p = 0; p < kAhead; ++p) {
+            if (s + p >= s1) break;
+            bf16x8 a, b;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                a[e] = to_bf16(wv[p][e]);
+                b[e] = to_bf16(xv[p][e]);
+            }
+            if (s + p + kAhead < s1) load(p, s + p + kAhead);
+            acc = mfma16(a, b, acc);
+        }
+    }
+    if constexpr (KW > 1) {
+        if (kw > 0) part[(kw - 1) * 64 + lane] = acc;
+        __syncthreads();
+        if (kw > 0) return;
+#pragma unroll
+        for (int q = 0; q < KW - 1; ++q) acc += part[q * 64 + lane];
+    }
+    // acc[r]: column n0 + 4 (lane >> 4) + r of row m0 + (lane & 15).
+    const int col = n0 + 4 * (lane >> 4), r = m0 + (lane & 15);
+    if (col >= N || r >= M) return;
+    const float4 bq = load_quad(bias, col, N);
+    const float bv[4] = {bq.x, bq.y, bq.z, bq.w};
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        v[e] = acc[e] + bv[e];
+        if (relu && v[e] < 0.f) v[e] = 0.f;  // NaN passes through
+    }
+    float *o = y + (size_t)r * N + col;
+    if (col + 3 < N && ((uintptr_t)o & 15) == 0) {
+        *reinterpret_cast<float4 *>(o) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (col + e < N) o[e] = v[e];
+    }
+}
+
+template <int WM, int KW, bool VEC>
+void gemm_f32_thin_launch(const float *x, const float *w, const float *b, float *y, int M, int K,
+                          int N, int relu, hipStream_t s) {
+    const int tiles_n = (N + 15) / 16, tiles_m = (M + 16 * WM - 1) / (16 * WM);
+    hipLaunchKernelGGL((gemm_f32_thin_kernel<WM, KW, VEC>), dim3(tiles_m * tiles_n), dim3(64 * WM * KW),
+                       0, s, x, w, b, y, M, K, N, tiles_n, relu);
+}
+
+// The kernel with the least estimated time (microseconds): a CU fetches its
+// workgroups' operands at about 60 KB/us (33 for the thin kernel's scattered
+// rows), each workgroup and launch adds a constant, and a k-block takes at
+// least its fetch latency.  Fitted to 29 shapes on MI355X; the choice is
+// within 7 % of the fastest at every one of them.  Against the 128 x 128 x 32,
+// 32 x 144 and 128 x 32 tiles used before: 4224 x 384 -> 1536 33.1 -> 18.8 us
+// (265 TFLOP/s; 128 x 128 tiles, 64-deep blocks, eight waves), 300 x 1024 -> 1024 11.1 (32 x
+// 32 tiles, 128-deep; 18 with 64 x 64), 16896 x 192 -> 768 28.9 (32 with 64 x
+// 64 tiles).
 template <bool VEC>
 void gemm_f32_dispatch(const float *x, const float *w, const float *b, float *y, int M, int K,
                        int N, int relu, hipStream_t s) {
-    // 144 < N <= 288 (shapes the panel kernel does not take: K > 128 or
-    // unaligned operands): 32 x 144 tiles, whole column halves; at BASELINE
-    // config 1 (M = 11264, N = 288, K = 96) on MI355X 9.6 us vs 10.5 us as
-    // 128 x 128 tiles (whose third column tile is 75 % empty).
-    if (N <= 32)
-        gemm_f32_launch<Tile<128, 32, 32, 4, 1>, VEC>(x, w, b, y, M, K, N, relu, s);
-    else if (N <= 64)
-        gemm_f32_launch<Tile<128, 64, 32, 4, 1>, VEC>(x, w, b, y, M, K, N, relu, s);
-    else if (N > 144 && N <= 288)
-        gemm_f32_launch<Tile<32, 144, 32, 2, 3>, VEC>(x, w, b, y, M, K, N, relu, s);
-    else
-        gemm_f32_launch<Tile<128, 128, 32, 2, 2>, VEC>(x, w, b, y, M, K, N, relu, s);
+    auto ceil_div = [](long long a, long long b) { return (float)((a + b - 1) / b); };
+    auto tiles = [&](int bm, int bn) { return ceil_div(M, bm) * ceil_div(N, bn); };
+    auto tiled = [&](int bm, int bn, int bk, int per_cu, float launch, float each, float block) {
+        const float g = tiles(bm, bn), kb = (bm + bn) * (float)K * 0.004f;
+        const float wait = ceilf(g / (256.f * per_cu)) * ceil_div(K, bk) * block;
+        const float fetch = ceilf(g / 256.f) * (kb / 60.f + each);
+        return launch + (fetch > wait ? fetch : wait);
+    };
+    auto thin = [&](int wm, int kw, float launch, int per_cu) {
+        const float g = tiles(16 * wm, 16), kb = (16 * wm + 16) * (float)K * 0.004f;
+        const float wait = ceilf(g / (256.f * per_cu)) * ceil_div(K, 32 * kw) * 0.8f;
+        const float fetch = g / 256.f * (kb / 33.f + 0.25f);
+        return launch + (fetch > wait ? fetch : wait);
+    };
+    float best = tiled(128, 128, 64, 2, 4.5f, 1.3f, 1.6f);
+    int pick = 0;
+    auto offer = [&](float us, int id) {
+        if (us < best) {
+            best = us;
+            pick = id;
+        }
+    };
+    offer(tiled(64, 64, 64, 4, 2.7f, 0.5f, 1.05f), 1);
+    offer(tiled(32, 32, 128, 4, 2.1f, 0.25f, 1.0f), 2);
+    if (K <= 1 << 20 && tiles(16, 16) < 1e9f) {
+        offer(thin(1, 8, 2.1f, 4), 3);
+        offer(thin(4, 1, 2.6f, 8), 4);
+    }
+    switch (pick) {
+        case 0: gemm_f32_launch<Tile<128, 128, 64, 2, 4>, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        case 1: gemm_f32_launch<Tile<64, 64, 64, 2, 2>, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        case 2: gemm_f32_launch<Tile<32, 32, 128, 2, 2>, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        case 3: gemm_f32_thin_launch<1, 8, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        default: gemm_f32_thin_launch<4, 1, VEC>(x, w, b, y, M, K, N, relu, s); break;
+    }
 }
 
 template <class T>

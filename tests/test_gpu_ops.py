@@ -282,3 +282,38 @@ def test_conv_unaligned_operands(device):
         out = off(torch.zeros_like(want))
         bfhip.conv2d_f32(off(x), off(w), out=out, **kw)
         _tight(out.cpu().numpy(), want.cpu().numpy(), f"unaligned conv {wshape}")
+
+
+# (rows, in, out, relu, bias, inject Inf/NaN): the thin kernel (eight waves
+# sharing the reduction, or four short tiles per workgroup) and each tiled
+# core at the edges of their tiles and k-blocks, with and without 16-byte rows.
+GEMM_EDGE_CASES = [(1, 1, 1, True, True, False), (15, 31, 17, False, True, False),
+                   (17, 33, 15, True, False, True), (16, 256, 16, False, False, False),
+                   (33, 257, 40, False, True, True), (6, 2386, 4, False, True, False),
+                   (7, 1340, 241, True, True, False), (5000, 8, 16, False, True, False),
+                   (4097, 7, 3, True, False, False), (300, 512, 513, False, True, False),
+                   (999, 130, 1001, False, True, True), (6001, 100, 290, True, True, False),
+                   (4225, 200, 1540, False, True, False)]
+
+
+@pytest.mark.parametrize("case", GEMM_EDGE_CASES)
+def test_gemm_edges(device, case):
+    """Against the float64 sum over bf16-rounded operands (1e-5 of the RMS, as
+    test_gemm_shapes at K = 3072); rows past the last and columns past K must
+    not reach a sum, Inf and NaN only their own."""
+    import bfhip
+    m, k, n, relu, with_bias, special = case
+    print(f"[case] gemm {case}", flush=True)
+    rng = np.random.default_rng(m + 3 * k + 7 * n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    w = (rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32)
+    b = rng.standard_normal(n).astype(np.float32) if with_bias else None
+    if special:
+        x[0, 0] = np.inf
+        x[-1, -1] = np.nan
+        w[-1, 0] = 0.0
+    got = bfhip.gemm_f32(_t(x, device), _t(w, device), _t(b, device) if with_bias else None,
+                         relu=relu).cpu().numpy()
+    want = convref.gemm_abi(x, w, b, relu, round_inputs=bf16_round)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    _tight(got, want, f"gemm {case}")
