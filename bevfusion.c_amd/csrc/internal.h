@@ -29,3 +29,9 @@ __attribute__((visibility("hidden"))) int transfusion_decode_launch(
     void *stream, const bf_detections **device_detections, char *error, size_t cap);
 
 }  // namespace bfhip
+
+// For tests: the largest feature plane, in bytes, that the sparse convolutions
+// gather through 32-bit buffer offsets (at most, and by default, 2 GiB - 1);
+// above it they read rows through 64-bit addresses.
+struct bf_cuda_lidar_backbone;
+extern "C" void bfhip_lidar_offset_limit(bf_cuda_lidar_backbone *backbone, unsigned bytes);

@@ -16,13 +16,12 @@
 //                counts and an in-order write pass that also clears the map
 //                (no atomics across workgroups); then a neighbour table from
 //                output to input;
-//   convolution  gather GEMM on the matrix cores: 32 output rows per wave,
-//                K = taps x input channels, each lane gathering its row's
-//                neighbour features as the A operand and the BN-folded
-//                weights [tap][co][ci] as B; taps no row of the wave uses
-//                are skipped; bias, residual add and ReLU fused in the
-//                epilogue.  The 5-channel input conv runs in fp32 on the
-//                vector units (its inputs are metric coordinates).
+//   convolution  gather GEMM on the matrix cores: K = taps x input channels,
+//                the rows' neighbour features against the BN-folded weights
+//                [tap][co][ci]; taps no row of a wave uses are skipped;
+//                bias, residual add and ReLU fused in the epilogue.  The
+//                5-channel input conv runs in fp32 on the vector units (its
+//                inputs are metric coordinates).
 // Precision: features and weights are kept as split fp16 pairs, x = hi + lo
 // with hi = fp16(x) and lo = fp16(x - hi), and every product is formed as
 // hi*Whi + lo*Whi + hi*Wlo on fp16 MFMAs with fp32 accumulation (the
@@ -33,7 +32,9 @@
 // RMS at its largest entries; the split keeps the encoder near fp32.
 // The output conv writes fp32 rows, gathered into the dense BEV.
 #include "bf_cuda_lidar.h"
+#include "gemm_core.h"
 #include "host_util.h"
+#include "internal.h"
 
 #include <algorithm>
 #include <climits>
@@ -47,7 +48,7 @@ using namespace bfhip;
 
 namespace {
 
-constexpr int kTaps = 27, kChunk = 8192, kRowsPerWave = 32, kRowsPerGroup = 4 * kRowsPerWave;
+constexpr int kTaps = 27, kChunk = 8192;
 constexpr int kEmpty = -1;
 constexpr float kBnEps = 1e-3f;
 
@@ -281,8 +282,7 @@ __global__ __launch_bounds__(256) void conv_input_kernel(const int *__restrict__
                                                          const float *__restrict__ feat,
                                                          const float *__restrict__ w,
                                                          const float *__restrict__ bias,
-                                                         _Float16 *__restrict__ out_hi,
-                                                         _Float16 *__restrict__ out_lo) {
+                                                         _Float16 *__restrict__ out) {
     const unsigned n = *count;
     for (unsigned j = blockIdx.x * 256 + threadIdx.x; j < n; j += gridDim.x * 256) {
         float acc[16];
@@ -309,8 +309,8 @@ __global__ __launch_bounds__(256) void conv_input_kernel(const int *__restrict__
         }
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            *(h8 *)&out_hi[(size_t)j * 16 + 8 * q] = hi[q];
-            *(h8 *)&out_lo[(size_t)j * 16 + 8 * q] = lo[q];
+            *(h8 *)&out[(size_t)j * 32 + 8 * q] = hi[q];  // a 16-channel row: hi words, lo words
+            *(h8 *)&out[(size_t)j * 32 + 16 + 8 * q] = lo[q];
         }
     }
 }
@@ -326,39 +326,31 @@ struct KOp {
     }
 };
 
-// Split fp16 feature planes of one level (rows x channels each).
-struct Feat {
-    _Float16 *hi, *lo;
+// Split fp16 features of one level: rows of C channels, each group of 32 (16
+// at C = 16) stored as its hi words, then its lo words, so that one 32-channel
+// step of a gather reads 128 contiguous bytes of a row.  As two planes, hi and
+// lo, it read two pieces of 64 bytes, half an L2 line each.
+typedef _Float16 *Feat;
+template <int C>
+struct FeatAt {
+    static constexpr int G = C < 32 ? C : 32;  // channels per group; lo words lie G after hi
+    __device__ static size_t hi(size_t row, int c) { return row * (2 * C) + (c / G) * (2 * G) + c % G; }
 };
 
-// LDS plan of one conv instantiation: the split weights of TPB taps, double
-// buffered, rows padded by 8 halves so the 16 lanes of a fragment read spread
-// over the banks; then the workgroup's neighbour table and active-tap list.
-// CO here is the workgroup's output columns; BUFS is 2 (double buffered) or 1.
-template <int CI, int CO, int BUFS = 2, int TPB = 1>
-struct ConvLds {
-    static constexpr int LD = CI + 8;        // halves per weight row in LDS
-    static constexpr int PLANE = CO * LD;    // halves per hi or lo plane
-    static constexpr int CHUNKS = 2 * CO * CI / 8;  // 16-byte pieces of one tap (hi + lo)
-    static constexpr int PER = (CHUNKS + 255) / 256;
-    static constexpr size_t W_BYTES = (size_t)BUFS * TPB * 2 * PLANE * sizeof(_Float16);
-    static constexpr size_t NBR_BYTES = (size_t)kRowsPerGroup * kTaps * sizeof(int);
-    static constexpr size_t BYTES = W_BYTES + NBR_BYTES + 32 * sizeof(int);
-};
-
-// Workgroup shape per layer width: output columns per workgroup and weight
-// buffers.  The 128-channel convs split their columns in two and stage one
-// tap at a time: 49 KB of LDS instead of 153 KB, so two workgroups share a
-// CU (the level-3 convs otherwise run one wave per SIMD), at the price of
-// gathering each feature row twice.  The 32-channel convs, with little math
-// per tap, stage two taps per barrier (TPB): 3% off the encoder on MI355X,
-// where three taps cost a wave per SIMD and lost, and two taps for the
-// 64-channel convs would do the same.
+// Workgroup shape per layer width: BM rows x all CO columns on WM x WN compute
+// waves, LW loader waves, S stages of one 32-channel step.  64 rows leave room
+// for two or more workgroups per CU; 128 rows read 36 % fewer weight bytes but
+// measured slower on every layer (128 channels, 30 427 rows: 76 us against 70;
+// 64 channels, 65 844 rows: 57 against 52).  Two to five stages are level.
 template <int CI, int CO>
 struct ConvShape {
-    static constexpr int COW = CI == 128 ? 64 : CO;
-    static constexpr int BUFS = CI == 128 ? 1 : 2;
-    static constexpr int TPB = CI == 32 ? 2 : 1;
+    static constexpr int BM = 64, WM = 2, WN = CO == 32 ? 1 : 2, LW = CO == 32 ? 2 : 4, S = 3;
+};
+template <int CO, int BM, int S>
+struct ConvLds {
+    static constexpr int A = BM * 64, B = CO * 64;           // halves: 32 channels' hi and lo words
+    static constexpr int STAGE = A + B;
+    static constexpr size_t BYTES = (size_t)S * STAGE * 2;
 };
 
 // Tap groups: a level with few rows has few 128-row workgroups, each walking
@@ -375,221 +367,235 @@ __device__ __forceinline__ int tap_groups(unsigned n, int launched) {
 }
 
 // Gather GEMM: out[r][co] = bias[co] + sum_t sum_ci in[nbr[r][t]][ci] w[t][co][ci]
-// (+ identity[r][co]) (ReLU), operands split as hi + lo.  A workgroup owns
-// 128 rows x COW of the CO columns (blockIdx.z picks the slice); each wave
-// 32 rows (two 16-row MFMA tiles).  Taps go in chunks of TPB per barrier.
-// BUFS = 1 stages one chunk's weights at a time (two barriers per chunk) to
-// leave room for more workgroups per CU.
+// (+ identity[r][co]) (ReLU), operands split as hi + lo.  A workgroup owns BM
+// rows x all CO columns, so every feature row is fetched once per tap that
+// uses it.  The rows' neighbour lists go to LDS and the taps some row uses are
+// listed; the reduction walks the list in 32-channel steps.  Loader waves
+// bring a step's rows and weights straight into LDS (buffer_load
+// ... lds: each lane's offset is its row's neighbour, out of range, hence
+// zero, where there is none), S - 1 steps ahead; the compute waves read
+// fragments and multiply (the wave-specialised pipeline of gemm_core.h).  A
+// wave skips the MFMAs of a tap none of its rows reaches.
 // blockIdx.y is the tap group; with several groups in effect the workgroup
-// writes its fp32 partial sums to `part` [group][row][co] instead.
-// Per workgroup: the rows' neighbour lists go to LDS and the taps some row
-// uses are listed; per chunk of listed taps the split weights [co][ci] are
-// staged in LDS (double buffered: the next chunk's weights are fetched into
-// registers while this chunk's MFMAs run) and every wave reads its B
-// fragments there, so a weight leaves L2 once per 128 rows instead of once
-// per 32.  A fragments are gathered straight from the feature rows, one chunk
-// ahead.  Taps are summed in list order whatever TPB is.  A wave skips
-// the MFMAs of a tap none of its rows reaches.  out32, when set, receives
-// fp32 rows instead of a split pair.
-template <int CI, int CO, int COW, int BUFS, int TPB>
-__global__ __launch_bounds__(256) void sparse_conv_kernel(
-    const int *__restrict__ nbr, const unsigned *__restrict__ count, int taps, Feat in,
-    const _Float16 *__restrict__ w_hi, const _Float16 *__restrict__ w_lo,
-    const float *__restrict__ bias, Feat identity, int relu, Feat out,
-    float *__restrict__ out32, float *__restrict__ part) {
-    using K = KOp<CI>;
-    using L = ConvLds<CI, COW, BUFS, TPB>;
-    typedef typename K::frag frag;
-    constexpr int CT = COW / 16, KC = CI / K::kb;
-    const int co0 = (int)blockIdx.z * COW;
-    extern __shared__ __align__(16) unsigned char smem[];
-    _Float16 *sw = reinterpret_cast<_Float16 *>(smem);  // [buffer][hi, lo][CO][LD]
-    int *snbr = reinterpret_cast<int *>(smem + L::W_BYTES);  // [row][kTaps]
-    int *stap = snbr + kRowsPerGroup * kTaps;                // [0] mask, [1] count, [2..] list
+// writes its fp32 partial sums to `part` [group][row][co] instead.  out32, when
+// set, receives fp32 rows instead of a split pair.
+// The weights are the MFMA's A operand, so a lane ends with four consecutive
+// columns of one row and stores each plane as 8 bytes.  Consecutive row blocks
+// run on one XCD: in cell order they share most of their neighbours' rows.
+template <int CI, int CO, int BM, int WM, int WN, int LW, int S>
+__global__ __launch_bounds__((WM * WN + LW) * 64) void sparse_conv_kernel(
+    const int *__restrict__ nbr, const unsigned *__restrict__ count,
+    const unsigned *__restrict__ in_count, int taps, Feat in, const _Float16 *__restrict__ w,
+    const float *__restrict__ bias, Feat identity, int relu, Feat out, float *__restrict__ out32,
+    float *__restrict__ part, unsigned dma_bytes) {
+    using L = ConvLds<CO, BM, S>;
+    constexpr int KC = CI / 32, kCompute = WM * WN, kThreads = (kCompute + LW) * 64;
+    constexpr int kRowsW = BM / WM, kColsW = CO / WN, FR = kRowsW / 16, FC = kColsW / 16;
+    constexpr int IA = BM * 8 / (64 * LW), IB = CO * 8 / (64 * LW), P = IA + IB;
+    static_assert(BM * 8 % (64 * LW) == 0 && CO * 8 % (64 * LW) == 0, "whole DMA instructions per loader wave");
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[L::BYTES];
+    __shared__ int snbr[BM * kTaps];
+    __shared__ unsigned smask[WM];        // taps used by each wave row
+    __shared__ int slist[kTaps + 1];      // active taps; last entry: their number
+    bf16 *ring = reinterpret_cast<bf16 *>(smem);
     const unsigned n = *count;
     const int groups = tap_groups(n, (int)gridDim.y), group = (int)blockIdx.y;
     if (group >= groups) return;  // whole workgroup: before any barrier
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
-    const int wrow = wave * kRowsPerWave;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool loader = wave >= kCompute;
+    const unsigned row_blocks = (n + BM - 1) / BM;
 
-    // 16-byte pieces of tap t's weights: piece c < CHUNKS/2 of the hi plane,
-    // the rest of the lo plane; row cc / (CI/8), halves k..k+7.
-    auto fetch = [&](int t, h8 (&reg)[L::PER]) {
+    // Loader lanes: LDS chunk q (16 bytes) belongs to row q / 8, in the slot
+    // order of dma_swizzle<64>: chunks 0-3 of a row are hi words, 4-7 lo.
+    int arow[IA];
+    uint32_t acol[IA], boff[IB];
+    if (loader) {
+        const int w0 = wave - kCompute;
 #pragma unroll
-        for (int q = 0; q < L::PER; ++q) {
-            const int c = tid + 256 * q;
-            if (c < L::CHUNKS) {
-                const int half = c >= L::CHUNKS / 2, cc = c - half * (L::CHUNKS / 2);
-                const _Float16 *src = (half ? w_lo : w_hi) + ((size_t)t * CO + co0) * CI +
-                                      (size_t)cc * 8;
-                reg[q] = *reinterpret_cast<const h8 *>(src);
-            }
+        for (int j = 0; j < IA; ++j) {
+            const int q = (j * LW + w0) * 64 + lane, r = q >> 3;
+            arow[j] = r * kTaps;
+            acol[j] = 16u * ((q & 7) ^ dma_swizzle<64>(r));
         }
-    };
-    auto stage = [&](int buf, const h8 (&reg)[L::PER]) {
 #pragma unroll
-        for (int q = 0; q < L::PER; ++q) {
-            const int c = tid + 256 * q;
-            if (c < L::CHUNKS) {
-                const int half = c >= L::CHUNKS / 2, cc = c - half * (L::CHUNKS / 2);
-                const int co = cc / (CI / 8), k = (cc % (CI / 8)) * 8;
-                *reinterpret_cast<h8 *>(sw + (size_t)(2 * buf + half) * L::PLANE + co * L::LD + k) =
-                    reg[q];
-            }
+        for (int j = 0; j < IB; ++j) {
+            const int q = (j * LW + w0) * 64 + lane, r = q >> 3;
+            boff[j] = (uint32_t)r * CI * 4u + 16u * ((q & 7) ^ dma_swizzle<64>(r));
         }
-    };
-    auto gather = [&](int t, frag (&ah)[2][KC], frag (&al)[2][KC], bool (&live)[2]) {
+    }
+    // Features past the 32-bit buffer offsets: the loaders read rows through
+    // 64-bit addresses and registers instead.
+    const unsigned rows_in = *in_count;
+    const bool wide = rows_in > dma_bytes / (CI * 4u);
+    const uint32_t feat_bytes = wide ? 0u : rows_in * (uint32_t)(CI * 4), w_bytes = (uint32_t)taps * CO * CI * 4;
+    const __amdgpu_buffer_rsrc_t ar = buffer_rsrc(in, feat_bytes), br = buffer_rsrc(w, w_bytes);
+
+    for (unsigned first = 0; first < row_blocks; first += gridDim.x) {
+        const unsigned here = min(gridDim.x, row_blocks - first);
+        if (blockIdx.x >= here) break;
+        const unsigned base = (first + xcd_swizzle((int)blockIdx.x, (int)here)) * BM;
+        if (tid < WM) smask[tid] = 0u;
+        __syncthreads();
+        // Neighbour lists to LDS: a wave takes two rows at a time (a row per
+        // half wave, lane = tap), all its loads first.
+        {
+            constexpr int kWaves = kThreads / 64, kRounds = BM / (2 * kWaves);
+            static_assert(BM % (2 * kWaves) == 0 && kRowsW % (2 * kRounds) == 0, "a wave's rows lie in one wave row");
+            const int t = lane & 31, r0 = wave * 2 * kRounds + (lane >> 5);
+            int v[kRounds];
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) {
-            const int src = snbr[(wrow + 16 * rt + col) * kTaps + t];
-            live[rt] = src >= 0;
+            for (int i = 0; i < kRounds; ++i) {
+                const unsigned r = base + r0 + 2 * i;
+                v[i] = t < taps && r < n ? nbr[(size_t)r * kTaps + t] : kEmpty;
+            }
+            unsigned used = 0;
 #pragma unroll
-            for (int kc = 0; kc < KC; ++kc) {
-                const int k0 = kc * K::kb + g * K::per_lane;
-                if (src >= 0) {
-                    ah[rt][kc] = *(const frag *)&in.hi[(size_t)src * CI + k0];
-                    al[rt][kc] = *(const frag *)&in.lo[(size_t)src * CI + k0];
+            for (int i = 0; i < kRounds; ++i) {
+                if (t < taps) snbr[(r0 + 2 * i) * kTaps + t] = v[i];
+                const unsigned long long live = __ballot(v[i] >= 0);
+                used |= (unsigned)live | (unsigned)(live >> 32);
+            }
+            if (lane == 0 && used) atomicOr(&smask[wave * 2 * kRounds / kRowsW], used);
+        }
+        __syncthreads();
+        if (tid < kTaps) {  // one wave: rank of each active tap
+            unsigned m = 0;
+#pragma unroll
+            for (int i = 0; i < WM; ++i) m |= smask[i];
+            if (m >> tid & 1u) slist[__popc(m & ((1u << tid) - 1u))] = tid;
+            if (tid == 0) slist[kTaps] = __popc(m);
+        }
+        __syncthreads();
+        // This group's part of the active-tap list: entries [t0, t0 + active).
+        const int listed = slist[kTaps], per = (listed + groups - 1) / groups;
+        const int t0 = min(listed, group * per), active = min(listed, t0 + per) - t0;
+        const int nk = active * KC;
+
+        if (loader) {
+            const int w0 = wave - kCompute;
+            // The next step's tap, 32-channel group and row offsets, read from
+            // LDS before the wait for a free stage.
+            int ti = 0, c = 0, tap = 0;
+            uint32_t aoff[IA];
+            auto prepare = [&]() {
+                if (c == 0) {
+                    tap = __builtin_amdgcn_readfirstlane(slist[min(t0 + ti, kTaps - 1)]);
+#pragma unroll
+                    for (int j = 0; j < IA; ++j) {
+                        const int src = snbr[arow[j] + tap];
+                        aoff[j] = src >= 0 ? (uint32_t)src * (CI * 4) + acol[j] : kDmaOutOfRange;
+                    }
+                }
+            };
+            auto issue = [&](int kt) {
+                bf16 *st = ring + (kt % S) * L::STAGE + w0 * 512;
+                if (wide) {
+#pragma unroll
+                    for (int j = 0; j < IA; ++j) {
+                        const int src = snbr[arow[j] + tap];
+                        const h8 none = {};
+                        reinterpret_cast<h8 *>(st + j * LW * 512)[lane] =
+                            src >= 0 ? *reinterpret_cast<const h8 *>(in + (size_t)src * (2 * CI) + 64 * c + acol[j] / 2) : none;
+                    }
                 } else {
-                    ah[rt][kc] = frag{};
-                    al[rt][kc] = frag{};
+#pragma unroll
+                    for (int j = 0; j < IA; ++j) dma16(ar, st + j * LW * 512, aoff[j], 128u * c);
                 }
+#pragma unroll
+                for (int j = 0; j < IB; ++j)
+                    dma16(br, st + L::A + j * LW * 512, boff[j], (uint32_t)tap * (CO * CI * 4) + 128u * c);
+                if (++c == KC) {
+                    c = 0;
+                    ++ti;
+                }
+                prepare();
+            };
+            prepare();
+#pragma unroll
+            for (int k = 0; k < S - 1; ++k)
+                if (k < nk) issue(k);
+            for (int kt = 0; kt < nk; ++kt) {
+                const int ahead = nk - 1 - kt;  // steps issued after this one
+                if (wide) wait_vmcnt<0>();
+                else DmaWait<S - 2>::template stages<P>(ahead < S - 2 ? ahead : S - 2);
+                lds_barrier();
+                if (kt + S - 1 < nk) issue(kt + S - 1);
             }
-        }
-    };
-
-    for (unsigned base = blockIdx.x * kRowsPerGroup; base < n; base += gridDim.x * kRowsPerGroup) {
-        if (tid == 0) stap[0] = 0;
-        __syncthreads();
-        unsigned used = 0;
-        for (int i = tid; i < kRowsPerGroup * taps; i += 256) {
-            const int r = i / taps, t = i - r * taps;
-            const int v = base + r < n ? nbr[(size_t)(base + r) * kTaps + t] : kEmpty;
-            snbr[r * kTaps + t] = v;
-            if (v >= 0) used |= 1u << t;
-        }
-        for (int o = 32; o > 0; o >>= 1) used |= __shfl_xor(used, o);
-        if (lane == 0) atomicOr(reinterpret_cast<unsigned *>(stap), used);
-        __syncthreads();
-        if (tid == 0) {
-            const unsigned m = (unsigned)stap[0];
-            int c = 0;
-            for (int t = 0; t < taps; ++t)
-                if (m >> t & 1u) stap[2 + c++] = t;
-            stap[1] = c;
-        }
-        __syncthreads();
-        // This group's part of the active-tap list: entries [first, last).
-        const int listed = stap[1], per = (listed + groups - 1) / groups;
-        const int first = min(listed, group * per), last = min(listed, first + per);
-        const int *list = stap + 2 + first;
-        const int active = last - first;
-
-        f32x4 acc[2][CT];
+        } else {
+            const int wm = wave / WN, wn = wave % WN, col = lane & 15, g = lane >> 4;
+            const int hi = 8 * (g ^ dma_swizzle<64>(col)), lo = 8 * ((4 + g) ^ dma_swizzle<64>(col));
+            const int arow0 = (wm * kRowsW + col) * 64, brow0 = L::A + (wn * kColsW + col) * 64;
+            const unsigned mine = smask[wm];
+            f32x4 acc[FC][FR];
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt)
+            for (int i = 0; i < FC; ++i)
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        // Chunk c holds list entries [c * TPB, min(active, c * TPB + TPB)).
-        const int chunks = (active + TPB - 1) / TPB;
-        h8 wreg[TPB][L::PER];
-        frag ah[TPB][2][KC], al[TPB][2][KC];
-        bool live[TPB][2] = {};
-        // Callers pass chunks that exist, so with TPB = 1 every entry does.
-        auto fetch_chunk = [&](int c) {
+                for (int j = 0; j < FR; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int kt = 0; kt < nk; ++kt) {
+                const int tap = __builtin_amdgcn_readfirstlane(slist[t0 + kt / KC]);
+                lds_barrier();
+                if (!(mine >> tap & 1u)) continue;  // wave-uniform
+                const bf16 *st = ring + (kt % S) * L::STAGE;
+                bf16x8 xh[FR], xl[FR];
 #pragma unroll
-            for (int u = 0; u < TPB; ++u)
-                if (TPB == 1 || c * TPB + u < active) fetch(list[c * TPB + u], wreg[u]);
-        };
-        auto stage_chunk = [&](int buf, int c) {
+                for (int j = 0; j < FR; ++j) {
+                    xh[j] = *reinterpret_cast<const bf16x8 *>(st + arow0 + j * 1024 + hi);
+                    xl[j] = *reinterpret_cast<const bf16x8 *>(st + arow0 + j * 1024 + lo);
+                }
 #pragma unroll
-            for (int u = 0; u < TPB; ++u)
-                if (TPB == 1 || c * TPB + u < active) stage(buf * TPB + u, wreg[u]);
-        };
-        auto gather_chunk = [&](int c, frag (&h)[TPB][2][KC], frag (&lo)[TPB][2][KC],
-                                bool (&lv)[TPB][2]) {
+                for (int i = 0; i < FC; ++i) {
+                    const bf16x8 wh = *reinterpret_cast<const bf16x8 *>(st + brow0 + i * 1024 + hi);
+                    const bf16x8 wl = *reinterpret_cast<const bf16x8 *>(st + brow0 + i * 1024 + lo);
 #pragma unroll
-            for (int u = 0; u < TPB; ++u)  // entries past the end keep lv false
-                if (TPB == 1 || c * TPB + u < active) gather(list[c * TPB + u], h[u], lo[u], lv[u]);
-        };
-        if (chunks) {
-            fetch_chunk(0);
-            stage_chunk(0, 0);
-            gather_chunk(0, ah, al, live);
-        }
-        __syncthreads();
-        for (int c = 0; c < chunks; ++c) {
-            const int buf = BUFS == 2 ? c & 1 : 0;
-            const bool more = c + 1 < chunks;
-            if (more) fetch_chunk(c + 1);
-            frag nh[TPB][2][KC], nl[TPB][2][KC];
-            bool nlive[TPB][2] = {};
-            if (more) gather_chunk(c + 1, nh, nl, nlive);
-#pragma unroll
-            for (int u = 0; u < TPB; ++u) {
-                // Wave-uniform: a tap none of the wave's rows reaches (or an
-                // entry past the list's end) adds nothing.
-                if (__ballot(live[u][0] || live[u][1])) {
-                    const _Float16 *bh_base = sw + (size_t)(2 * (buf * TPB + u)) * L::PLANE;
-                    const _Float16 *bl_base = bh_base + L::PLANE;
-#pragma unroll
-                    for (int kc = 0; kc < KC; ++kc) {
-                        const int k0 = kc * K::kb + g * K::per_lane;
-#pragma unroll
-                        for (int ct = 0; ct < CT; ++ct) {
-                            const int wo = (16 * ct + col) * L::LD + k0;
-                            const frag bh = *(const frag *)&bh_base[wo];
-                            const frag bl = *(const frag *)&bl_base[wo];
-#pragma unroll
-                            for (int rt = 0; rt < 2; ++rt) {
-                                acc[rt][ct] = K::mfma(al[u][rt][kc], bh, acc[rt][ct]);
-                                acc[rt][ct] = K::mfma(ah[u][rt][kc], bl, acc[rt][ct]);
-                                acc[rt][ct] = K::mfma(ah[u][rt][kc], bh, acc[rt][ct]);
-                            }
-                        }
+                    for (int j = 0; j < FR; ++j) {
+                        acc[i][j] = mfma16_f16(wh, xl[j], acc[i][j]);
+                        acc[i][j] = mfma16_f16(wl, xh[j], acc[i][j]);
+                        acc[i][j] = mfma16_f16(wh, xh[j], acc[i][j]);
                     }
                 }
             }
-            if (more) {
-                if (BUFS == 1) __syncthreads();  // every wave is done with this chunk's weights
-                stage_chunk(BUFS == 2 ? buf ^ 1 : 0, c + 1);
+            // acc[i][j][e]: column 16 i + 4 g + e of row 16 j + col of the wave.
 #pragma unroll
-                for (int u = 0; u < TPB; ++u)
+            for (int i = 0; i < FC; ++i) {
+                const int co = wn * kColsW + 16 * i + 4 * g;
+                const float4 b = *reinterpret_cast<const float4 *>(bias + co);
 #pragma unroll
-                    for (int rt = 0; rt < 2; ++rt) {
-                        live[u][rt] = nlive[u][rt];
-#pragma unroll
-                        for (int kc = 0; kc < KC; ++kc) {
-                            ah[u][rt][kc] = nh[u][rt][kc];
-                            al[u][rt][kc] = nl[u][rt][kc];
-                        }
-                    }
-            }
-            __syncthreads();
-        }
-        const unsigned row0 = base + wrow;
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct) {
-            const int co = co0 + 16 * ct + col;
-            const float b = bias[co];
-#pragma unroll
-            for (int rt = 0; rt < 2; ++rt)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const unsigned r = row0 + 16 * rt + 4 * g + j;
+                for (int j = 0; j < FR; ++j) {
+                    const unsigned r = base + wm * kRowsW + 16 * j + col;
                     if (r >= n) continue;
-                    const size_t at = (size_t)r * CO + co;
+                    const size_t at = (size_t)r * CO + co, fa = FeatAt<CO>::hi(r, co);
+                    float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
                     if (groups > 1) {
-                        part[((size_t)group * kSplitRows + r) * CO + co] = acc[rt][ct][j];
+                        *reinterpret_cast<float4 *>(part + (size_t)group * kSplitRows * CO + at) =
+                            make_float4(v[0], v[1], v[2], v[3]);
                         continue;
                     }
-                    float v = acc[rt][ct][j] + b;
-                    if (identity.hi) v += (float)identity.hi[at] + (float)identity.lo[at];
-                    if (relu) v = fmaxf(v, 0.0f);
-                    if (out32) out32[at] = v;
-                    else split_store(v, out.hi + at, out.lo + at);
+                    v[0] += b.x; v[1] += b.y; v[2] += b.z; v[3] += b.w;
+                    if (identity) {
+                        const h4 ih = *reinterpret_cast<const h4 *>(identity + fa);
+                        const h4 il = *reinterpret_cast<const h4 *>(identity + fa + FeatAt<CO>::G);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] += (float)ih[e] + (float)il[e];
+                    }
+                    if (relu)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = fmaxf(v[e], 0.0f);
+                    if (out32) {
+                        *reinterpret_cast<float4 *>(out32 + at) = make_float4(v[0], v[1], v[2], v[3]);
+                        continue;
+                    }
+                    h4 oh, ol;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        oh[e] = (_Float16)v[e];
+                        ol[e] = (_Float16)(v[e] - (float)oh[e]);
+                    }
+                    *reinterpret_cast<h4 *>(out + fa) = oh;
+                    *reinterpret_cast<h4 *>(out + fa + FeatAt<CO>::G) = ol;
                 }
+            }
         }
-        __syncthreads();  // LDS is rewritten by the next row group
+        __syncthreads();  // LDS is rewritten by the next row block
     }
 }
 
@@ -608,10 +614,11 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(
         float v = 0.0f;
         for (int gi = 0; gi < groups; ++gi) v += part[(size_t)gi * kSplitRows * CO + e];
         v += bias[co];
-        if (identity.hi) v += (float)identity.hi[e] + (float)identity.lo[e];
+        const size_t fa = FeatAt<CO>::hi(e / CO, co);
+        if (identity) v += (float)identity[fa] + (float)identity[fa + FeatAt<CO>::G];
         if (relu) v = fmaxf(v, 0.0f);
         if (out32) out32[e] = v;
-        else split_store(v, out.hi + e, out.lo + e);
+        else split_store(v, out + fa, out + fa + FeatAt<CO>::G);
     }
 }
 
@@ -652,8 +659,9 @@ __global__ __launch_bounds__(256) void sparse_conv_split_kernel(
             for (int kc = 0; kc < KC; ++kc) {
                 const int k0 = kc * K::kb + g * K::per_lane;
                 if (src >= 0) {
-                    f.ah[rt][kc] = *(const frag *)&in.hi[(size_t)src * CI + k0];
-                    f.al[rt][kc] = *(const frag *)&in.lo[(size_t)src * CI + k0];
+                    const _Float16 *row = in + FeatAt<CI>::hi(src, k0);
+                    f.ah[rt][kc] = *(const frag *)row;
+                    f.al[rt][kc] = *(const frag *)(row + FeatAt<CI>::G);
                 } else {
                     f.ah[rt][kc] = frag{};
                     f.al[rt][kc] = frag{};
@@ -730,10 +738,11 @@ __global__ __launch_bounds__(256) void sparse_conv_split_kernel(
             if (row >= n) continue;
             const size_t at = (size_t)row * CO + co;
             float v = part[0][r][co] + part[1][r][co] + part[2][r][co] + part[3][r][co] + bias[co];
-            if (identity.hi) v += (float)identity.hi[at] + (float)identity.lo[at];
+            const size_t fa = FeatAt<CO>::hi(row, co);
+            if (identity) v += (float)identity[fa] + (float)identity[fa + FeatAt<CO>::G];
             if (relu) v = fmaxf(v, 0.0f);
             if (out32) out32[at] = v;
-            else split_store(v, out.hi + at, out.lo + at);
+            else split_store(v, out + fa, out + fa + FeatAt<CO>::G);
         }
         __syncthreads();  // LDS is rewritten by the next row group
     }
@@ -782,6 +791,7 @@ struct Conv {
 
 struct bf_cuda_lidar_backbone {
     size_t batches, capacity, resident_bytes;
+    unsigned dma_bytes;  // largest feature plane the convs address with 32-bit offsets
     Grid lv[5];
     long long cells[5];
     int max_chunks;
@@ -879,8 +889,18 @@ int build(bf_cuda_lidar_backbone *n, const bf_model *m, char *error, size_t cap)
             std::vector<float> lo(t.size());
             for (size_t i = 0; i < t.size(); ++i)
                 lo[i] = t[i] - (float)(_Float16)t[i];
-            o.w = pa.add_f16(t);
-            o.w_lo = pa.add_f16(lo);
+            if (sp.ci < 32) {  // two planes
+                o.w = pa.add_f16(t);
+                o.w_lo = pa.add_f16(lo);
+            } else {  // per 32 input channels: hi words, lo words (as the features)
+                std::vector<float> both(2 * t.size());
+                for (size_t i = 0; i < t.size(); ++i) {
+                    const size_t at = i / 32 * 64 + i % 32;
+                    both[at] = t[i];
+                    both[at + 32] = lo[i];
+                }
+                o.w = o.w_lo = pa.add_f16(both);
+            }
         }
         o.b = pa.add_f32(bf);
         offs.push_back(o);
@@ -946,8 +966,7 @@ int build(bf_cuda_lidar_backbone *n, const bf_model *m, char *error, size_t cap)
     if (!hip_ok(hipMemset(n->marks, 0, mark_bytes), error, cap, "clear LiDAR mark map"))
         return 0;
     for (int i = 0; i < 3; ++i) {
-        n->feat[i].hi = (_Float16 *)(a + o_feat[i]);
-        n->feat[i].lo = n->feat[i].hi + n->capacity * 128;
+        n->feat[i] = (_Float16 *)(a + o_feat[i]);
     }
     n->out32 = (float *)(a + o_out);
     n->part = (float *)(a + o_part);
@@ -963,8 +982,7 @@ unsigned row_blocks(size_t capacity, int rows_per_block) {
 }
 
 void launch_conv(const bf_cuda_lidar_backbone *n, const Conv &c, const unsigned *count,
-                 Feat in, Feat identity, int relu, Feat out, float *out32, hipStream_t s) {
-    const unsigned blocks = row_blocks(n->capacity, kRowsPerGroup);
+                 const unsigned *in_count, Feat in, Feat identity, int relu, Feat out, float *out32, hipStream_t s) {
     const unsigned split_blocks =
         (unsigned)std::max<size_t>(1, std::min<size_t>(16384, (n->capacity + 31) / 32));
 #define BF_SPLIT(CI, CO)                                                                       \
@@ -980,10 +998,10 @@ void launch_conv(const bf_cuda_lidar_backbone *n, const Conv &c, const unsigned 
     if (c.ci == CI && c.co == CO) {                                                            \
         using S = ConvShape<CI, CO>;                                                           \
         const int groups = CI >= 64 ? kTapGroups : 1;                                          \
-        sparse_conv_kernel<CI, CO, S::COW, S::BUFS, S::TPB>                                            \
-            <<<dim3(blocks, groups, CO / S::COW), 256, ConvLds<CI, S::COW, S::BUFS, S::TPB>::BYTES,    \
-               s>>>(n->nbr, count, c.taps, in, c.w_hi, c.w_lo, c.bias, identity, relu, out,    \
-                    out32, n->part);                                                           \
+        sparse_conv_kernel<CI, CO, S::BM, S::WM, S::WN, S::LW, S::S>                           \
+            <<<dim3(row_blocks(n->capacity, S::BM), groups), (S::WM * S::WN + S::LW) * 64, 0, s>>>( \
+                n->nbr, count, in_count, c.taps, in, c.w_hi, c.bias, identity, relu, out, out32,    \
+                n->part, n->dma_bytes);                                                        \
         if (groups > 1)                                                                        \
             split_reduce_kernel<CO><<<1024, 256, 0, s>>>(count, groups, n->part, c.bias,       \
                                                          identity, relu, out, out32);          \
@@ -1021,8 +1039,8 @@ void forward_impl(bf_cuda_lidar_backbone *n, const bf_coord4 *coords, const floa
     subm_neighbors_kernel<<<nbr_blocks(n), 256, 0, s>>>(coords, n->counts, n->lv[0], n->grid[0],
                                                         n->nbr);
     conv_input_kernel<<<rb, 256, 0, s>>>(n->nbr, n->counts, feats, n->input.w32, n->input.bias,
-                                         n->feat[0].hi, n->feat[0].lo);
-    const Feat none{nullptr, nullptr};
+                                         n->feat[0]);
+    const Feat none = nullptr;
     int x = 0;
     const bf_coord4 *level_coords = coords;
     for (int st = 0; st < 4; ++st) {
@@ -1030,7 +1048,7 @@ void forward_impl(bf_cuda_lidar_backbone *n, const bf_coord4 *coords, const floa
         if (st) {
             strided_sites(n, n->down[st - 1], st - 1, level_coords, s);
             const int y = (x + 1) % 3;
-            launch_conv(n, n->down[st - 1], cnt, n->feat[x], none, 1, n->feat[y], nullptr, s);
+            launch_conv(n, n->down[st - 1], cnt, cnt - 1, n->feat[x], none, 1, n->feat[y], nullptr, s);
             x = y;
             level_coords = n->coords[st];
             subm_neighbors_kernel<<<nbr_blocks(n), 256, 0, s>>>(level_coords, cnt, n->lv[st],
@@ -1038,14 +1056,14 @@ void forward_impl(bf_cuda_lidar_backbone *n, const bf_coord4 *coords, const floa
         }
         for (int blk = 0; blk < 2; ++blk) {
             const int y = (x + 1) % 3, z = (x + 2) % 3;
-            launch_conv(n, n->res[st][blk][0], cnt, n->feat[x], none, 1, n->feat[y], nullptr, s);
-            launch_conv(n, n->res[st][blk][1], cnt, n->feat[y], n->feat[x], 1, n->feat[z], nullptr,
+            launch_conv(n, n->res[st][blk][0], cnt, cnt, n->feat[x], none, 1, n->feat[y], nullptr, s);
+            launch_conv(n, n->res[st][blk][1], cnt, cnt, n->feat[y], n->feat[x], 1, n->feat[z], nullptr,
                         s);
             x = z;
         }
     }
     strided_sites(n, n->out, 3, level_coords, s);
-    launch_conv(n, n->out, n->counts + 4, n->feat[x], none, 1, none, n->out32, s);
+    launch_conv(n, n->out, n->counts + 4, n->counts + 3, n->feat[x], none, 1, none, n->out32, s);
     const size_t dense_tiles = (size_t)n->lv[4].b * (((size_t)n->cells[4] / n->lv[4].b + 63) / 64);
     dense_kernel<<<(unsigned)std::min<size_t>(16384, dense_tiles), 256, 0, s>>>(
         n->grid[4], n->lv[4], n->out32, dense);
@@ -1071,20 +1089,6 @@ extern "C" void bf_cuda_lidar_backbone_destroy(bf_cuda_lidar_backbone *n) {
 extern "C" size_t bf_cuda_lidar_backbone_resident_bytes(const bf_cuda_lidar_backbone *n) {
     return n ? n->resident_bytes : 0;
 }
-
-namespace {
-
-template <int CI, int CO>
-int allow_lds(char *error, size_t cap) {
-    using S = ConvShape<CI, CO>;
-    return hip_ok(hipFuncSetAttribute(
-                      reinterpret_cast<const void *>(&sparse_conv_kernel<CI, CO, S::COW, S::BUFS, S::TPB>),
-                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                      (int)ConvLds<CI, S::COW, S::BUFS, S::TPB>::BYTES),
-                  error, cap, "set LiDAR conv LDS size");
-}
-
-}  // namespace
 
 extern "C" int bf_cuda_lidar_backbone_create(const bf_model *model, size_t batches, size_t d,
                                              size_t h, size_t w, size_t capacity,
@@ -1116,9 +1120,8 @@ extern "C" int bf_cuda_lidar_backbone_create(const bf_model *model, size_t batch
         }
         n->cells[l] = (long long)n->lv[l].b * n->lv[l].d * n->lv[l].h * n->lv[l].w;
     }
-    if (!allow_lds<32, 32>(error, cap) || !allow_lds<32, 64>(error, cap) ||
-        !allow_lds<64, 64>(error, cap) || !allow_lds<64, 128>(error, cap) ||
-        !allow_lds<128, 128>(error, cap) || !build(n, model, error, cap)) {
+    n->dma_bytes = INT_MAX;
+    if (!build(n, model, error, cap)) {
         bf_cuda_lidar_backbone_destroy(n);
         return 0;
     }
@@ -1146,4 +1149,8 @@ extern "C" int bf_cuda_lidar_backbone_forward_count_device(bf_cuda_lidar_backbon
         return fail(error, cap, "invalid device-count HIP LiDAR buffers");
     forward_impl(n, coords, feats, count, 0u, dense, reinterpret_cast<hipStream_t>(stream));
     return launch_ok(error, cap, "HIP LiDAR launch");
+}
+
+extern "C" void bfhip_lidar_offset_limit(bf_cuda_lidar_backbone *n, unsigned bytes) {
+    n->dma_bytes = std::min(bytes, (unsigned)INT_MAX);
 }

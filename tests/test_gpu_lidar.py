@@ -17,6 +17,8 @@ synthetic frame.  Bars:
     their eager launches (no memset or allocation inside).
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -164,6 +166,25 @@ def test_lidar_backbone_small_grid(device, lidar_path):
     want2 = _backbone_oracle(lidar_path, half, feats[: len(half)], 41, 96, 96)
     got2 = net.forward(_t(half, device), _t(feats[: len(half)], device), len(half)).cpu().numpy()
     _check_bev(got2, want2, "41x96x96 half")
+    net.close()
+
+
+@pytest.mark.parametrize("sites", [1, 2, 63, 64, 65, 129, 4000])
+def test_lidar_conv_row_blocks(device, lidar_path, sites):
+    """Site counts at the edges of the convs' 64-row blocks (one row, a full
+    block, one over), and the same forward with every feature row gathered
+    through a 64-bit address: bit-identical."""
+    print(f"[case] lidar conv row blocks {sites}", flush=True)
+    coords = clustered_sites(17, 12 * sites, 41, 64, 72)[:sites]
+    feats = np.random.default_rng(sites).standard_normal((len(coords), 5)).astype(np.float32)
+    with bfhip.Model(lidar_path) as m:
+        net = bfhip.LidarBackbone(m, 1, 41, 64, 72, 40000)
+    c, f = _t(coords, device), _t(feats, device)
+    got = net.forward(c, f, len(coords)).cpu().numpy()
+    _check_bev(got, _backbone_oracle(lidar_path, coords, feats, 41, 64, 72), f"{len(coords)} sites")
+    net.lib.bfhip_lidar_offset_limit.argtypes = [ctypes.c_void_p, ctypes.c_uint]
+    net.lib.bfhip_lidar_offset_limit(net.handle, 0)
+    assert np.array_equal(net.forward(c, f, len(coords)).cpu().numpy(), got)
     net.close()
 
 
