@@ -118,6 +118,19 @@ using SFuser = DmaTile<128, 256, 64, 2, 4, 3, true>;
 constexpr int kLoaders = 4;
 constexpr int kFuserIn = 336, kFuserPad = 384;
 
+// One conv of the stage: the small-grid tiles where the map is small, else
+// the tuned tile T, on the wave-specialised core if it has three stages and
+// on the plain one if two.
+template <class T, int K, class Epi>
+void bev_conv(const ConvLayer &l, const bf16 *a, int c0, const bf16 *b, int c1, const Epi &epi,
+              hipStream_t s) {
+    if (run_conv_few<K>(l, a, c0, b, c1, epi, s)) return;
+    if constexpr (T::kStages > 2)
+        run_conv_spec<T, K, kLoaders>(l, a, c0, b, c1, epi, s);
+    else
+        run_conv_dma<T, K>(l, a, c0, b, c1, epi, s);
+}
+
 }  // namespace
 
 struct bf_cuda_bev_stage {
@@ -248,20 +261,19 @@ void forward_impl(bf_cuda_bev_stage *s, const float *input, float *spatial, floa
     const int H = (int)s->h, W = (int)s->w, H2 = H / 2, W2 = W / 2;
     const size_t hw = (size_t)H * W;
     pack_nhwc(input, s->in, 1, kFuserIn, H * W, st, true, kFuserPad);
-    run_conv_spec<SFuser, 3, kLoaders>(s->L[kFuser], s->in, kFuserPad, nullptr, 0,
-                                       nhwc_to(s->L[kFuser], s->pa, true), st);
+    bev_conv<SFuser, 3>(s->L[kFuser], s->in, kFuserPad, nullptr, 0,
+                        nhwc_to(s->L[kFuser], s->pa, true), st);
     bf16 *cur = s->pa, *nxt = s->pb;
     for (int l = 0; l < 6; ++l) {
         const ConvLayer &c = s->L[kBlock0 + l];
-        run_conv_spec<SFull, 3, kLoaders>(c, cur, c.ci, nullptr, 0, nhwc_to(c, nxt, true), st);
+        bev_conv<SFull, 3>(c, cur, c.ci, nullptr, 0, nhwc_to(c, nxt, true), st);
         std::swap(cur, nxt);
     }
     const ConvLayer &d0 = s->L[kDeblock0];
-    run_conv_dma<DFull, 1>(d0, cur, 128, nullptr, 0, out_to(d0, s->s0, spatial, 1, true), st);
+    bev_conv<DFull, 1>(d0, cur, 128, nullptr, 0, out_to(d0, s->s0, spatial, 1, true), st);
     for (int l = 0; l < 6; ++l) {
         const ConvLayer &c = s->L[kBlock1 + l];
-        run_conv_spec<SHalf, 3, kLoaders>(c, cur, l == 0 ? 128 : 256, nullptr, 0,
-                                          nhwc_to(c, nxt, true), st);
+        bev_conv<SHalf, 3>(c, cur, l == 0 ? 128 : 256, nullptr, 0, nhwc_to(c, nxt, true), st);
         std::swap(cur, nxt);
     }
     // deblock.1: [H2 W2 x 256] x [1024 x 256]^T, scattered to 2x resolution
@@ -273,12 +285,11 @@ void forward_impl(bf_cuda_bev_stage *s, const float *input, float *spatial, floa
                                         (int)hw},
                            m, 1024, 256, st);
     const ConvLayer &sc = s->L[kShared];
-    run_conv_spec<SFull, 3, kLoaders>(sc, s->s0, 256, s->s1, 256, out_to(sc, s->sh, shared, 0, true),
-                                      st);
+    bev_conv<SFull, 3>(sc, s->s0, 256, s->s1, 256, out_to(sc, s->sh, shared, 0, true), st);
     const ConvLayer &hm = s->L[kHeatMid];
-    run_conv_spec<SFull, 3, kLoaders>(hm, s->sh, 128, nullptr, 0, nhwc_to(hm, s->pa, true), st);
+    bev_conv<SFull, 3>(hm, s->sh, 128, nullptr, 0, nhwc_to(hm, s->pa, true), st);
     const ConvLayer &ho = s->L[kHeatOut];
-    run_conv_dma<DHalf, 3>(ho, s->pa, 128, nullptr, 0, out_to(ho, nullptr, heatmap, 0, true), st);
+    bev_conv<DHalf, 3>(ho, s->pa, 128, nullptr, 0, out_to(ho, nullptr, heatmap, 0, true), st);
 }
 
 }  // namespace

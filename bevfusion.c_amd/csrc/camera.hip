@@ -105,6 +105,7 @@ constexpr int kDsLoaders = 5;
 template <class Epi>
 void conv_256(const ConvLayer &l, const bf16 *a, int c0, const bf16 *b, int c1, const Epi &epi,
               hipStream_t s) {
+    if (run_conv_few<3>(l, a, c0, b, c1, epi, s)) return;
     if (use_s256(l))
         run_conv_spec<S256, 3, kS256Loaders>(l, a, c0, b, c1, epi, s);
     else
@@ -112,7 +113,8 @@ void conv_256(const ConvLayer &l, const bf16 *a, int c0, const bf16 *b, int c1, 
 }
 template <class Epi>
 void conv_fpn1(const ConvLayer &l, const bf16 *in, const Epi &epi, hipStream_t s) {
-    run_conv_spec<S64, 3, kS64Loaders>(l, in, 256, nullptr, 0, epi, s);
+    if (!run_conv_few<3>(l, in, 256, nullptr, 0, epi, s))
+        run_conv_spec<S64, 3, kS64Loaders>(l, in, 256, nullptr, 0, epi, s);
 }
 // dtransform.3 and .6 as jobs: the forward runs each in one launch with a
 // lateral's lower half (neck_impl), the other entry points and the probes
@@ -138,7 +140,8 @@ void conv_dt2(const ConvLayer &l, const bf16 *in, const Epi &epi, hipStream_t s)
 }
 template <class Epi>
 void conv_dn6(const ConvLayer &l, const bf16 *in, const Epi &epi, hipStream_t s) {
-    run_conv_dma<D256, 1>(l, in, 256, nullptr, 0, epi, s);
+    if (!run_conv_few<1>(l, in, 256, nullptr, 0, epi, s))
+        run_conv_dma<D256, 1>(l, in, 256, nullptr, 0, epi, s);
 }
 template <class Epi>
 void conv_ds0(const ConvLayer &l, const bf16 *in, const Epi &epi, hipStream_t s) {

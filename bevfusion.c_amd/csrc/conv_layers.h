@@ -102,6 +102,33 @@ void run_conv_spec(const ConvLayer &l, const bf16 *a, int c0, const bf16 *b, int
     launch_gemm_spec<T>(al, bl, epi, g.M, l.co, g.K, s);
 }
 
+// Limit of the small-grid rule (few_tile_rows) for the 3x3 and 1x1 convs: one
+// tile per CU (their reductions are long, so a full round of small tiles
+// still wins).  Measured on MI355X (pixels, Ci -> Co: 64 x 128 spec tile ->
+// the rule's, us): 324, 256 -> 256 16.5 -> 8.1; 1024, 256 -> 256 16.8 -> 8.3;
+// 2025, 256 -> 256 16.7 -> 9.8; 4096, 512 -> 128 27.9 -> 15.2; 8100, 128 ->
+// 128 11.1 -> 9.2.
+constexpr int kFewConv = 256;
+
+// Runs the conv on a small-grid tile if its grid is one; returns whether it did.
+template <int K, class Epi>
+bool run_conv_few(const ConvLayer &l, const bf16 *a, int c0, const bf16 *b, int c1, const Epi &epi,
+                  hipStream_t s) {
+    const int rows = few_tile_rows(l.n * l.oh * l.ow, l.co, kFewConv, kFewConv);
+    if (!rows) return false;
+    const auto run = [&](auto r) {
+        constexpr int R = decltype(r)::value;
+        if (c0 % 128 == 0 && c1 % 128 == 0)
+            run_conv_spec<FewTile128<R>, K, few_loaders<FewTile128<R>>()>(l, a, c0, b, c1, epi, s);
+        else
+            run_conv_spec<FewTile64<R>, K, few_loaders<FewTile64<R>>()>(l, a, c0, b, c1, epi, s);
+    };
+    if (rows == 16) run(std::integral_constant<int, 16>{});
+    else if (rows == 32) run(std::integral_constant<int, 32>{});
+    else run(std::integral_constant<int, 64>{});
+    return true;
+}
+
 // The same convs as jobs of gemm_pair_kernel (gemm_core.h), for a launch
 // shared with an independent layer.
 template <class T, int KH, int KW, class Src, class Epi>

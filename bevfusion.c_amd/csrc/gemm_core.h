@@ -786,6 +786,31 @@ inline void launch_gemm_spec(const ALoad &al, const BLoad &bl, const Epi &epi, i
                        K, tiles_n);
 }
 
+// ------------------------------------------------------- grids of few tiles
+// The tuned tiles of the layers are sized for full grids (one or more tiles
+// per CU).  On a small input such a grid is a handful of workgroups, each of
+// which walks its whole reduction at its own CU's fetch rate with two or three
+// stages in flight while most of the chip idles: the time then is the bytes
+// one workgroup reads, whatever the input's size.  There a layer runs on the
+// smallest of three tiles 64 columns wide whose grid still fits: 16, 32 or 64
+// rows on the wave-specialised core with four loader waves and as many stages
+// as the LDS holds, 128-deep k-steps where the operands allow them (half the
+// barriers; twice the bytes a loader wave keeps in flight).  `limit` bounds
+// the tiles of 16 and 32 rows, `limit64` those of 64; 0: the tuned tile.
+// Every tile sums k in the same order, so the choice does not change results.
+template <int ROWS>
+using FewTile128 = DmaTile<ROWS, 64, 128, ROWS == 16 ? 1 : 2, ROWS == 16 ? 4 : 2, ROWS == 64 ? 4 : 6, true>;
+template <int ROWS>
+using FewTile64 = DmaTile<ROWS, 64, 64, ROWS == 16 ? 1 : 2, ROWS == 16 ? 4 : 2, ROWS == 64 ? 4 : 8, true>;
+template <class T>
+constexpr int few_loaders() { return T::BM * T::BK >= 4 * kWave * 8 ? 4 : 2; }
+inline int few_tile_rows(int M, int N, int limit, int limit64) {
+    const int64_t cols = (N + 63) / 64;
+    if ((M + 15) / 16 * cols <= limit) return 16;
+    if ((M + 31) / 32 * cols <= limit) return 32;
+    return (M + 63) / 64 * cols <= limit64 ? 64 : 0;
+}
+
 // ============================================ two independent GEMMs, one launch
 // A GEMM (or implicit-GEMM conv) as a job of gemm_pair_kernel: the tile
 // instance, its loaders and epilogue, on one of the three cores.

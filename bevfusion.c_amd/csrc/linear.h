@@ -74,6 +74,17 @@ inline LinearTile pick_linear_tile(int N, int K) {
     return K <= 96 ? kK32 : kK64;
 }
 
+// Limits of the small-grid rule (few_tile_rows) for these layers.  Measured on
+// MI355X with rotating weights (M x N x K: tuned tile -> the rule's, us):
+// 56 x 1152 x 384 5.6 -> 3.4, 56 x 384 x 1536 7.0 -> 5.3, 16 x 3072 x 768 8.8
+// -> 4.2, 704 x 192 x 768 8.8 -> 4.2, 704 x 576 x 192 4.5 -> 3.2, 352 x 1536 x
+// 384 6.9 -> 4.2, 4224 x 192 x 768 9.0 -> 5.2.  The reductions are short, so a
+// grid that fills the chip pays for its repeated operand reads: 16-row tiles
+// cross 32-row ones near 200 tiles (216 of them: 5.7 vs 4.8 us; 198: 3.8 vs
+// 3.9), and 64-row tiles, two to a CU, hold to 512 (408: 5.9 us vs 7.6 tuned;
+// 528: 6.1 vs 5.8).
+constexpr int kFewLinear = 200, kFewLinear64 = 512;
+
 // Buffer-resource offsets are 32-bit: both operands must span < 2 GiB, rows
 // start 16-byte aligned and K is a multiple of 8 (true of every layer here;
 // checked by the callers' contexts at create).
@@ -85,6 +96,16 @@ inline bool linear_operands_ok(const void *x, const void *w, int M, int N, int K
 template <class Epi>
 inline void linear_f16(const bf16 *x, const bf16 *w, int M, int N, int K, const Epi &epi,
                         hipStream_t s) {
+    if (N % 64 == 0)
+        switch (few_tile_rows(M, N, kFewLinear, kFewLinear64)) {
+            case 16: return linear_spec<FewTile128<16>, 4>(x, w, M, N, K, epi, s);
+            case 32: return linear_spec<FewTile64<32>, 4>(x, w, M, N, K, epi, s);
+            case 64:
+                if (K >= 768 && (M + 63) / 64 * (N / 64) <= 256)
+                    return linear_spec<DmaTile<64, 64, 128, 2, 2, 3, true>, 4>(x, w, M, N, K, epi, s);
+                return linear_spec<FewTile64<64>, 4>(x, w, M, N, K, epi, s);
+            default: break;
+        }
     switch (pick_linear_tile(N, K)) {
         case kK32: linear_tile<DmaTile<64, 64, 32, 2, 2, 2, true>>(x, w, M, N, K, epi, s); break;
         case kK64: linear_tile<DmaTile<64, 64, 64, 2, 2, 2, true>>(x, w, M, N, K, epi, s); break;

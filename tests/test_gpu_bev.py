@@ -53,6 +53,15 @@ def test_bev_stage_matches_oracle(bev_path, hw, device):
     stage.close()
 
 
+# The convs' tile follows the grid: 128 outputs run 16-row tiles up to 2048
+# pixels, 32-row to 4096, 64-row to 8192, the tuned ones beyond (half of each
+# at 256 outputs and half resolution).  Either side of each line, odd rows left
+# over in the last tile.
+@pytest.mark.parametrize("hw", [(38, 54), (46, 46), (62, 66), (66, 64), (90, 92)])
+def test_bev_stage_small_grids(bev_path, hw, device):
+    test_bev_stage_matches_oracle(bev_path, hw, device)
+
+
 def test_bev_stage_graph_replays(bev_path, device):
     import torch
     x = bfw.synthetic_bev(6, 36, 52)

@@ -52,6 +52,24 @@ def test_fpn_matches_oracle(device, tmp_models, b, h, w):
     assert_close(f0.cpu().numpy(), r0, "fpn0")
 
 
+# One camera and several take different tiles (16, 32, 64 rows or the tuned
+# one, by the grid), which sum in the same order: camera k of the batch is
+# bit-identical to its own forward.
+@pytest.mark.parametrize("b,h,w", [(6, 6, 9), (4, 16, 17), (5, 24, 40), (6, 32, 88)])
+def test_neck_tiles_agree_across_batches(device, tmp_models, b, h, w):
+    import torch
+    from bfhip import bfw
+    path = tmp_models("fan_in", 1)
+    levels = [_t(a, device) for a in _swin_like(b, h, w)]
+    depth = _t(bfw.synthetic_depth(2, b, 8 * h, 8 * w), device)
+    many = _neck(path, b, h, w).neck_forward(*levels, depth)
+    one = _neck(path, 1, h, w)
+    for k in range(b):
+        got = one.neck_forward(*[x[k:k + 1].contiguous() for x in levels], depth[k:k + 1].contiguous())
+        for g, m in zip(got, many):
+            assert torch.equal(g[0], m[k]), f"camera {k} of {b}x{h}x{w}"
+
+
 @pytest.mark.parametrize("b,h,w", [(1, 2, 3), (2, 3, 5), (1, 32, 88)])
 def test_depth_head_matches_oracle(device, tmp_models, b, h, w):
     import oracle

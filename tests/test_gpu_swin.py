@@ -50,6 +50,24 @@ def test_swin_matches_oracle(device, tmp_models, shape):
         assert_close(g, r, f"swin {shape} output{i}")
 
 
+# One image and several take different linear and merge tiles (16, 32, 64 rows
+# or the tuned one, by the grid), which sum in the same order: image k of the
+# batch is bit-identical to its own forward.
+@pytest.mark.parametrize("shape", [(3, 32, 32), (4, 64, 96), (3, 96, 352), (5, 128, 352)])
+def test_swin_tiles_agree_across_batches(device, tmp_models, shape):
+    import bfhip
+    import torch
+    from bfhip import bfw
+    b, h, w = shape
+    x = torch.from_numpy(bfw.synthetic_images(3, b, h, w)).to(device)
+    with bfhip.Model(tmp_models("fan_in", 1)) as m:
+        many, one = bfhip.Swin(m, b, h, w), bfhip.Swin(m, 1, h, w)
+    outs = many.forward(x)
+    for k in range(b):
+        for g, o in zip(one.forward(x[k:k + 1].contiguous()), outs):
+            assert torch.equal(g[0], o[k]), f"image {k} of {shape}"
+
+
 def test_swin_baseline_init_matches_oracle(device, tmp_models):
     """BASELINE.json weight init (N(0,0.02)) at one production camera."""
     from bfhip import bfw
