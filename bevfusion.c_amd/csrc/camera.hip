@@ -53,6 +53,9 @@ struct bf_cuda_camera_neck {
 
 namespace {
 
+// Maps with few pixels run the 3x3 256-channel convs and depthnet.6 on the
+// small-grid tiles (run_conv_few; neck and downsample of one 85 x 8 camera 179
+// -> 120 us); the rest is for full grids.
 // Tiles from sweeps of both cores on these shapes (MI355X).  DMA-fed: 64 x 128
 // for the 256-channel 3x3 convs at 32x88 below full camera batch and the
 // depthnet.6 1x1; the level-0 and level-1 3x3 convs, dtransform.6 and the
@@ -74,6 +77,12 @@ using S256 = DmaTile<160, 128, 64, 2, 4, 3, true>;
 constexpr int kS256Loaders = 4;
 inline bool use_s256(const ConvLayer &l) {
     return l.co == 256 && 2 * ((l.n * l.oh * l.ow + 159) / 160) >= 128;
+}
+// Between the small-grid tiles and those: 64-row tiles on the same pipeline
+// while they are at most one per CU (8192 pixels at 256 outputs).
+using SMid = DmaTile<64, 128, 64, 2, 2, 6, true>;
+inline bool use_smid(const ConvLayer &l) {
+    return l.co == 256 && 2 * ((l.n * l.oh * l.ow + 63) / 64) <= 256;
 }
 // fpn_convs.1 at level 1 (M = 4224, two loader waves) and dtransform.6 (32
 // input channels, so 32-deep k-steps) on the wave-specialised pipeline:
@@ -106,7 +115,9 @@ template <class Epi>
 void conv_256(const ConvLayer &l, const bf16 *a, int c0, const bf16 *b, int c1, const Epi &epi,
               hipStream_t s) {
     if (run_conv_few<3>(l, a, c0, b, c1, epi, s)) return;
-    if (use_s256(l))
+    if (use_smid(l))
+        run_conv_spec<SMid, 3, kS256Loaders>(l, a, c0, b, c1, epi, s);
+    else if (use_s256(l))
         run_conv_spec<S256, 3, kS256Loaders>(l, a, c0, b, c1, epi, s);
     else
         run_conv_dma<D256, 3>(l, a, c0, b, c1, epi, s);

@@ -14,8 +14,9 @@
 // stage-3 fc1; stage-1 fc1 (1584 tiles of 64 x 128) as 32-deep k-steps in
 // three stages, whose 36 KiB of LDS let four workgroups share a CU (1.55
 // rounds instead of 2.06 at three: 18.9 vs 19.7 us).  (N, K)
-// identifies the layer, so the table holds for any camera count; other shapes
-// take the 64-deep default.
+// identifies the layer, so the table holds for any camera count whose grid
+// the small-grid rule below does not take (stage-2 proj is the one layer of six
+// full-size cameras that it does); other shapes take the 64-deep default.
 //
 // Four layers measured faster on the wave-specialised pipeline
 // (gemm_spec_kernel: loader waves issue every DMA, so the compute waves'
