@@ -115,6 +115,27 @@ def test_voxelize_bit_exact(device, points, max_voxels):
         assert _voxel_gpu(vox, np.zeros((0, 5), np.float32), device)[2] == 0
 
 
+@pytest.mark.parametrize("points", [16384, 16385, 16391, 40001])
+def test_voxelize_crowded(device, points):
+    """Voxels of ten to thousands of points on both sides of the split into two
+    insertion launches, descending through the cloud and shuffled: the kept
+    points are each voxel's first ones."""
+    rng = np.random.default_rng(points)
+    cells = np.minimum(rng.geometric(0.08, points), 60)
+    pts = np.zeros((points, 5), np.float32)
+    pts[:, 0] = (cells + 0.5) * 0.075
+    pts[:, 1:3] = rng.uniform(0.0, 0.07, (points, 2))
+    pts[:, 3:] = rng.random((points, 2))
+    pts[::17, 0] = np.nan  # dropped
+    o = oracle.Oracle("port")
+    with bfhip.Voxelizer(bfhip.voxel_config(160000), 40001) as vox:
+        for cloud in (pts, pts[np.argsort(-cells, kind="stable")]):
+            vx, oc, on, _ = o.voxelize(cloud, oracle.voxel_config(160000))
+            gc, gm, n = _voxel_gpu(vox, cloud, device)
+            assert n == len(oc) and np.array_equal(gc, oc)
+            assert np.array_equal(gm, o.mean_vfe(vx, on))
+
+
 def test_voxelize_known_answers(device):
     cfg = bfhip.voxel_config(2, max_points=2)
     p = np.array([[0.01, 0.01, 0.01, 1, 0], [10.0, 0.0, 0.0, 2, 0], [0.02, 0.02, 0.02, 3, 0],
