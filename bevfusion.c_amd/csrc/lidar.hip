@@ -253,19 +253,31 @@ __global__ __launch_bounds__(256) void compact_write_kernel(
     __syncthreads();
     unsigned idx = base + inc - c;
     for (int w2 = 0; w2 < wave; ++w2) idx += part[w2];
-    while (bits) {
+    if (!bits) return;
+    // The group's first cell, decoded once; its other cells are steps along x.
+    // Three 64-bit divisions per site took about half of this kernel's time
+    // (100 000-point clouds on MI355X: 13.9 us per level; now 7.6).
+    long long q = w * 32;
+    int x0 = (int)(q % g.w);
+    q /= g.w;
+    int y = (int)(q % g.h);
+    q /= g.h;
+    int z = (int)(q % g.d), n = (int)(q / g.d);
+    while (bits && idx < capacity) {
         const int b = __ffs(bits) - 1;
         bits &= bits - 1;
-        if (idx < capacity) {
-            long long q = w * 32 + b;
-            grid[q] = (int)idx;
-            const int x = (int)(q % g.w);
-            q /= g.w;
-            const int y = (int)(q % g.h);
-            q /= g.h;
-            const int z = (int)(q % g.d);
-            coords[idx] = bf_coord4{(int)(q / g.d), z, y, x};
+        while (x0 + b >= g.w) {
+            x0 -= g.w;
+            if (++y == g.h) {
+                y = 0;
+                if (++z == g.d) {
+                    z = 0;
+                    ++n;
+                }
+            }
         }
+        grid[w * 32 + b] = (int)idx;
+        coords[idx] = bf_coord4{n, z, y, x0 + b};
         ++idx;
     }
 }
@@ -353,7 +365,7 @@ struct ConvLds {
     static constexpr size_t BYTES = (size_t)S * STAGE * 2;
 };
 
-// Tap groups: a level with few rows has few 128-row workgroups, each walking
+// Tap groups: a level with few rows has few 64-row workgroups, each walking
 // every tap in turn while most CUs idle, so up to kTapGroups workgroups share
 // a row block, each taking a contiguous part of its active-tap list and
 // writing fp32 partial sums; split_reduce_kernel adds them in group order.
