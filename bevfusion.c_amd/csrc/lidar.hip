@@ -35,6 +35,7 @@
 #include "gemm_core.h"
 #include "host_util.h"
 #include "internal.h"
+#include "tap_walk.h"
 
 #include <algorithm>
 #include <climits>
@@ -478,20 +479,19 @@ __global__ __launch_bounds__((WM * WN + LW) * 64) void sparse_conv_kernel(
             if (tid == 0) slist[kTaps] = __popc(m);
         }
         __syncthreads();
-        // This group's part of the active-tap list: entries [t0, t0 + active).
-        const int listed = slist[kTaps], per = (listed + groups - 1) / groups;
-        const int t0 = min(listed, group * per), active = min(listed, t0 + per) - t0;
-        const int nk = active * KC;
+        // This group's part of the active-tap list.
+        TapWalk walk(slist[kTaps], groups, group);
+        const int t0 = walk.next, nk = (walk.end - t0) * KC;
 
         if (loader) {
             const int w0 = wave - kCompute;
             // The next step's tap, 32-channel group and row offsets, read from
             // LDS before the wait for a free stage.
-            int ti = 0, c = 0, tap = 0;
+            int tap = 0;
             uint32_t aoff[IA];
             auto prepare = [&]() {
-                if (c == 0) {
-                    tap = __builtin_amdgcn_readfirstlane(slist[min(t0 + ti, kTaps - 1)]);
+                if (walk.starts_tap()) {
+                    tap = __builtin_amdgcn_readfirstlane(slist[walk.next]);
 #pragma unroll
                     for (int j = 0; j < IA; ++j) {
                         const int src = snbr[arow[j] + tap];
@@ -501,6 +501,7 @@ __global__ __launch_bounds__((WM * WN + LW) * 64) void sparse_conv_kernel(
             };
             auto issue = [&](int kt) {
                 bf16 *st = ring + (kt % S) * L::STAGE + w0 * 512;
+                const int c = walk.c;
                 if (wide) {
 #pragma unroll
                     for (int j = 0; j < IA; ++j) {
@@ -516,10 +517,7 @@ __global__ __launch_bounds__((WM * WN + LW) * 64) void sparse_conv_kernel(
 #pragma unroll
                 for (int j = 0; j < IB; ++j)
                     dma16(br, st + L::A + j * LW * 512, boff[j], (uint32_t)tap * (CO * CI * 4) + 128u * c);
-                if (++c == KC) {
-                    c = 0;
-                    ++ti;
-                }
+                walk.step(KC);
                 prepare();
             };
             prepare();

@@ -64,3 +64,24 @@ def clustered_sites(seed, n, d, h, w):
     uniq = np.unique(pts, axis=0)
     rng.shuffle(uniq)
     return np.concatenate([np.zeros((len(uniq), 1), np.int32), uniq.astype(np.int32)], 1)
+
+
+def run_host_check(source, tmp_path):
+    """Compiles tests/<source> with hipcc, runs its host code (nothing runs on
+    a GPU) and returns what it printed."""
+    import pathlib
+    import shutil
+    import subprocess
+
+    import pytest
+    root = pathlib.Path(__file__).resolve().parents[1]
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not pathlib.Path(hipcc).exists():
+        pytest.skip("hipcc not available")
+    exe = tmp_path / "check"
+    subprocess.run([hipcc, "--offload-arch=gfx950", "-O1", "-std=c++17",
+                    f"-I{root / 'bevfusion.c_amd' / 'csrc'}", f"-I{root / 'include'}",
+                    str(root / "tests" / source), "-o", str(exe)], check=True, capture_output=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stdout + out.stderr
+    return out.stdout
