@@ -409,6 +409,9 @@ __device__ __forceinline__ void gemm_reg_block(ALoad &al, BLoad &bl, const Epi &
 }
 
 // Host launcher: one workgroup per output tile.
+// Whether a launch holds the grid: HIP takes at most 2^32 - 1 threads along x.
+inline bool launch_fits(long long workgroups, int threads) { return workgroups <= 0xffffffffll / threads; }
+
 template <class T, class ALoad, class BLoad, class Epi>
 inline void launch_gemm(const ALoad &al, const BLoad &bl, const Epi &epi, int M, int N, int K,
                         hipStream_t stream) {

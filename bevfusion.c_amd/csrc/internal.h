@@ -35,3 +35,9 @@ __attribute__((visibility("hidden"))) int transfusion_decode_launch(
 // above it they read rows through 64-bit addresses.
 struct bf_cuda_lidar_backbone;
 extern "C" void bfhip_lidar_offset_limit(bf_cuda_lidar_backbone *backbone, unsigned bytes);
+
+// For tests: the kernel that bf_cuda_gemm_f32 runs on these operands
+// (GemmRoute in ops.hip; pointers for their alignment only, -1: refused as too
+// large).
+extern "C" int bfhip_gemm_route(const float *x, const float *w, const float *b, const float *y,
+                                int rows, int in_f, int out_f);

@@ -9,6 +9,7 @@
 #include "bf_cuda_ops.h"
 #include "conv_core.h"
 #include "conv_direct.h"
+#include "internal.h"
 
 #include <climits>
 
@@ -138,16 +139,19 @@ __global__ __launch_bounds__(kPanelThreads) void gemm_f32_panel_kernel(
     }
 }
 
-// The panel kernel for (M, K, N), or false when the shape is not one it takes.
-bool gemm_f32_panel(const float *x, const float *w, const float *b, float *y, int M, int K, int N,
+// Whether the panel kernel takes the shape.
+bool gemm_f32_panel_takes(const float *x, const float *w, const float *b, const float *y, int M,
+                          int K, int N) {
+    return M >= kPanelMinRows && K <= 128 && !(K & 3) && !(N & 3) && N > 144 &&
+           N <= 2 * 16 * kPanelMaxFrags && (long long)N * K * 4 < (1ll << 31) && aligned16(x) &&
+           aligned16(w) && aligned16(y) && (!b || aligned16(b)) &&
+           panel_lds_bytes(N, (K + 31) / 32) <= 65536;
+}
+
+void gemm_f32_panel(const float *x, const float *w, const float *b, float *y, int M, int K, int N,
                     int relu, hipStream_t s) {
-    if (M < kPanelMinRows || K > 128 || (K & 3) || (N & 3) || N <= 144 || N > 2 * 16 * kPanelMaxFrags ||
-        (long long)N * K * 4 >= (1ll << 31) || !aligned16(x) || !aligned16(w) || !aligned16(y) ||
-        (b && !aligned16(b)))
-        return false;
     const int ks = (K + 31) / 32;
     const size_t lds = panel_lds_bytes(N, ks);
-    if (lds > 65536) return false;
     const dim3 grid((M + kPanelRows - 1) / kPanelRows, 2);
     const int nc = panel_cols(N);
     switch (ks) {
@@ -156,7 +160,6 @@ bool gemm_f32_panel(const float *x, const float *w, const float *b, float *y, in
         case 3: hipLaunchKernelGGL(gemm_f32_panel_kernel<3>, grid, dim3(kPanelThreads), lds, s, x, w, b, y, M, K, N, nc, relu); break;
         default: hipLaunchKernelGGL(gemm_f32_panel_kernel<4>, grid, dim3(kPanelThreads), lds, s, x, w, b, y, M, K, N, nc, relu); break;
     }
-    return true;
 }
 
 // Few or thin outputs: one wave per 16 x 16 output tile, no LDS staging.  The
@@ -261,53 +264,72 @@ void gemm_f32_thin_launch(const float *x, const float *w, const float *b, float 
                        0, s, x, w, b, y, M, K, N, tiles_n, relu);
 }
 
-// The kernel with the least estimated time (microseconds): a CU fetches its
-// workgroups' operands at about 60 KB/us (33 for the thin kernel's scattered
-// rows), each workgroup and launch adds a constant, and a k-block takes at
-// least its fetch latency.  Fitted to 29 shapes on MI355X; the choice is
-// within 7 % of the fastest at every one of them.  Against the 128 x 128 x 32,
-// 32 x 144 and 128 x 32 tiles used before: 4224 x 384 -> 1536 33.1 -> 18.8 us
-// (265 TFLOP/s; 128 x 128 tiles, 64-deep blocks, eight waves), 300 x 1024 -> 1024 11.1 (32 x
-// 32 tiles, 128-deep; 18 with 64 x 64), 16896 x 192 -> 768 28.9 (32 with 64 x
-// 64 tiles).
-template <bool VEC>
-void gemm_f32_dispatch(const float *x, const float *w, const float *b, float *y, int M, int K,
-                       int N, int relu, hipStream_t s) {
-    auto ceil_div = [](long long a, long long b) { return (float)((a + b - 1) / b); };
+// The kernel with the least estimated time (microseconds) of those whose grid a
+// launch holds: a CU fetches its workgroups' operands at about 60 KB/us (33 for
+// the thin kernel's scattered rows), each workgroup and launch adds a constant,
+// and a k-block takes at least its fetch latency.  Fitted to 29 shapes on
+// MI355X; the choice is within 7 % of the fastest at every one of them.  Against
+// the 128 x 128 x 32, 32 x 144 and 128 x 32 tiles used before: 4224 x 384 ->
+// 1536 33.1 -> 18.8 us (265 TFLOP/s; 128 x 128 tiles, 64-deep blocks, eight
+// waves), 300 x 1024 -> 1024 11.1 (32 x 32 tiles, 128-deep; 18 with 64 x 64),
+// 16896 x 192 -> 768 28.9 (32 with 64 x 64 tiles).  From some 10^9 rows only the
+// four-wave 128 x 128 tile has few enough threads; kGemmNone: none has.
+enum GemmRoute { kGemmNone = -1, kGemm128, kGemm64, kGemm32, kGemmThinSplit, kGemmThinRows, kGemmWide, kGemmPanel };
+using Gemm128 = Tile<128, 128, 64, 2, 4>;
+using Gemm64 = Tile<64, 64, 64, 2, 2>;
+using Gemm32 = Tile<32, 32, 128, 2, 2>;
+using GemmWide = Tile<128, 128, 32, 2, 2>;
+
+GemmRoute gemm_route(int M, int K, int N) {
+    auto ceil_div = [](long long a, long long b) { return (a + b - 1) / b; };
     auto tiles = [&](int bm, int bn) { return ceil_div(M, bm) * ceil_div(N, bn); };
     auto tiled = [&](int bm, int bn, int bk, int per_cu, float launch, float each, float block) {
-        const float g = tiles(bm, bn), kb = (bm + bn) * (float)K * 0.004f;
-        const float wait = ceilf(g / (256.f * per_cu)) * ceil_div(K, bk) * block;
+        const float g = (float)tiles(bm, bn), kb = (bm + bn) * (float)K * 0.004f;
+        const float wait = ceilf(g / (256.f * per_cu)) * (float)ceil_div(K, bk) * block;
         const float fetch = ceilf(g / 256.f) * (kb / 60.f + each);
         return launch + (fetch > wait ? fetch : wait);
     };
     auto thin = [&](int wm, int kw, float launch, int per_cu) {
-        const float g = tiles(16 * wm, 16), kb = (16 * wm + 16) * (float)K * 0.004f;
-        const float wait = ceilf(g / (256.f * per_cu)) * ceil_div(K, 32 * kw) * 0.8f;
+        const float g = (float)tiles(16 * wm, 16), kb = (16 * wm + 16) * (float)K * 0.004f;
+        const float wait = ceilf(g / (256.f * per_cu)) * (float)ceil_div(K, 32 * kw) * 0.8f;
         const float fetch = g / 256.f * (kb / 33.f + 0.25f);
         return launch + (fetch > wait ? fetch : wait);
     };
-    float best = tiled(128, 128, 64, 2, 4.5f, 1.3f, 1.6f);
-    int pick = 0;
-    auto offer = [&](float us, int id) {
-        if (us < best) {
+    float best = INFINITY;
+    GemmRoute pick = kGemmNone;
+    auto offer = [&](GemmRoute id, int bm, int bn, int threads, float us) {
+        if (us < best && launch_fits(tiles(bm, bn), threads)) {
             best = us;
             pick = id;
         }
     };
-    offer(tiled(64, 64, 64, 4, 2.7f, 0.5f, 1.05f), 1);
-    offer(tiled(32, 32, 128, 4, 2.1f, 0.25f, 1.0f), 2);
-    if (K <= 1 << 20 && tiles(16, 16) < 1e9f) {
-        offer(thin(1, 8, 2.1f, 4), 3);
-        offer(thin(4, 1, 2.6f, 8), 4);
+    offer(kGemm128, 128, 128, Gemm128::kThreads, tiled(128, 128, 64, 2, 4.5f, 1.3f, 1.6f));
+    offer(kGemm64, 64, 64, Gemm64::kThreads, tiled(64, 64, 64, 4, 2.7f, 0.5f, 1.05f));
+    offer(kGemm32, 32, 32, Gemm32::kThreads, tiled(32, 32, 128, 4, 2.1f, 0.25f, 1.0f));
+    if (K <= 1 << 20 && tiles(16, 16) < 1000000000) {
+        offer(kGemmThinSplit, 16, 16, 8 * kWave, thin(1, 8, 2.1f, 4));
+        offer(kGemmThinRows, 64, 16, 4 * kWave, thin(4, 1, 2.6f, 8));
     }
-    switch (pick) {
-        case 0: gemm_f32_launch<Tile<128, 128, 64, 2, 4>, VEC>(x, w, b, y, M, K, N, relu, s); break;
-        case 1: gemm_f32_launch<Tile<64, 64, 64, 2, 2>, VEC>(x, w, b, y, M, K, N, relu, s); break;
-        case 2: gemm_f32_launch<Tile<32, 32, 128, 2, 2>, VEC>(x, w, b, y, M, K, N, relu, s); break;
-        case 3: gemm_f32_thin_launch<1, 8, VEC>(x, w, b, y, M, K, N, relu, s); break;
-        default: gemm_f32_thin_launch<4, 1, VEC>(x, w, b, y, M, K, N, relu, s); break;
+    if (pick == kGemmNone && launch_fits(tiles(128, 128), GemmWide::kThreads)) pick = kGemmWide;
+    return pick;
+}
+
+template <bool VEC>
+void gemm_f32_dispatch(GemmRoute route, const float *x, const float *w, const float *b, float *y,
+                       int M, int K, int N, int relu, hipStream_t s) {
+    switch (route) {
+        case kGemm128: gemm_f32_launch<Gemm128, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        case kGemm64: gemm_f32_launch<Gemm64, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        case kGemm32: gemm_f32_launch<Gemm32, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        case kGemmThinSplit: gemm_f32_thin_launch<1, 8, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        case kGemmThinRows: gemm_f32_thin_launch<4, 1, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        default: gemm_f32_launch<GemmWide, VEC>(x, w, b, y, M, K, N, relu, s); break;
     }
+}
+
+GemmRoute gemm_f32_route(const float *x, const float *w, const float *b, const float *y, int M,
+                         int K, int N) {
+    return gemm_f32_panel_takes(x, w, b, y, M, K, N) ? kGemmPanel : gemm_route(M, K, N);
 }
 
 template <class T>
@@ -490,11 +512,18 @@ extern "C" int bf_cuda_gemm_f32(const float *input, const float *weight, const f
     if (((long long)rows + 127) / 128 * ((out_f + 31LL) / 32) > INT_MAX)
         return fail(error, cap, "HIP GEMM is too large");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (gemm_f32_panel(input, weight, bias, output, rows, in_f, out_f, relu, s))
-        ;  // short reduction: one pass per row panel
+    const GemmRoute route = gemm_f32_route(input, weight, bias, output, rows, in_f, out_f);
+    if (route == kGemmNone) return fail(error, cap, "HIP GEMM is too large");
+    if (route == kGemmPanel)  // short reduction: one pass per row panel
+        gemm_f32_panel(input, weight, bias, output, rows, in_f, out_f, relu, s);
     else if ((in_f & 3) == 0 && aligned16(input) && aligned16(weight))
-        gemm_f32_dispatch<true>(input, weight, bias, output, rows, in_f, out_f, relu, s);
+        gemm_f32_dispatch<true>(route, input, weight, bias, output, rows, in_f, out_f, relu, s);
     else
-        gemm_f32_dispatch<false>(input, weight, bias, output, rows, in_f, out_f, relu, s);
+        gemm_f32_dispatch<false>(route, input, weight, bias, output, rows, in_f, out_f, relu, s);
     return launch_ok(error, cap, "HIP GEMM launch");
+}
+
+extern "C" int bfhip_gemm_route(const float *x, const float *w, const float *b, const float *y,
+                                int rows, int in_f, int out_f) {
+    return gemm_f32_route(x, w, b, y, rows, in_f, out_f);
 }

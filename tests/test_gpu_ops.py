@@ -317,3 +317,18 @@ def test_gemm_edges(device, case):
     want = convref.gemm_abi(x, w, b, relu, round_inputs=bf16_round)
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
     _tight(got, want, f"gemm {case}")
+
+
+def test_gemm_very_many_rows(device):
+    """2^30 + 77 rows: tiles of 64 rows would need more threads than a launch
+    holds.  One product per element, so the result is exact."""
+    import bfhip
+    import torch
+    m = 2 ** 30 + 77
+    x = torch.randn(m, 1, device=device)
+    w = torch.full((1, 1), 0.5, device=device)
+    out = torch.empty(m, 1, device=device)
+    print(f"[case] gemm {m}x1 -> 1", flush=True)
+    bfhip.gemm_f32(x, w, out=out)
+    for a in range(0, m, 2 ** 28):
+        assert torch.equal(out[a:a + 2 ** 28], x[a:a + 2 ** 28].bfloat16().float() * 0.5), a
