@@ -369,8 +369,8 @@ inline float direct_estimate(const DirectConv &d, int batches) {
 }
 
 // Fills in the rectangle, channel block and tile counts of tile T with the
-// least estimate; false when no rectangle's patch fits or an offset could
-// leave 32 bits.  quads: whole quads of slots per block (WV); flat: rectangles
+// least estimate; false when no rectangle's patch fits, an offset could leave
+// 32 bits or the grid is more than a launch holds.  quads: whole quads of slots per block (WV); flat: rectangles
 // of whole pixel quads (XV).
 template <class T>
 inline bool direct_plan(DirectConv &d, int batches, int kh, bool quads, bool flat, float *us) {
@@ -397,7 +397,7 @@ inline bool direct_plan(DirectConv &d, int batches, int kh, bool quads, bool fla
         if (o < 1 || 32ll * o * d.IH * d.IW >= 1ll << 30 || 32ll * o * wrow >= 1ll << 30) continue;
         d.TH = th; d.TW = tw; d.O = o; d.patch_w = (int)pw; d.patch = (int)patch;
         const long long ty = (d.OH + th - 1) / th, tx = (d.OW + tw - 1) / tw;
-        if (ty * tx * d.tiles_c * batches > 0x7fffffff) continue;
+        if (!launch_fits(ty * tx * d.tiles_c * batches, T::kThreads)) continue;
         d.tiles_y = (int)ty; d.tiles_x = (int)tx;
         const float e = direct_estimate<T>(d, batches);
         if (*us < 0.f || e < *us) {

@@ -6,6 +6,7 @@
 
 #include "bevfusion.h"
 #include "bf_cuda_depth_raster.h"
+#include "bf_cuda_ops.h"
 #include "bf_cuda_transfusion.h"
 #include "bf_cuda_voxel.h"
 
@@ -41,3 +42,8 @@ extern "C" void bfhip_lidar_offset_limit(bf_cuda_lidar_backbone *backbone, unsig
 // large).
 extern "C" int bfhip_gemm_route(const float *x, const float *w, const float *b, const float *y,
                                 int rows, int in_f, int out_f);
+
+// For tests: the kernel that bf_cuda_conv2d_f32 runs (ConvRoute in ops.hip) and
+// the threads of its launch (0 for the gather core).
+extern "C" int bfhip_conv_route(const bf_cuda_conv2d_desc *desc, const float *x, const float *w,
+                                const float *y, unsigned long long *threads);

@@ -370,42 +370,42 @@ void conv_direct_launch(const DirectConv &d, int batches, bool vec, bool flat, h
     }
 }
 
-// Plans every tile and launches the one with the least estimate; false when
-// none takes the shape.
-bool conv_direct_best(const DirectConv &d, int batches, int kh, bool wv, bool flat, hipStream_t s) {
-    using Big = DirectTile<128, 160, 2, 2, 8, 9, 1>;
-    using Mid = DirectTile<64, 128, 2, 2, 4, 9, 1>;
-    using Low = DirectTile<32, 64, 1, 4, 4, 9, 1>;
-    using Min = DirectTile<32, 32, 2, 2, 4, 9, 1>;
-    struct Choice { DirectConv d; float us; int tile; bool vec; } best{d, -1.f, -1, false};
-    auto offer = [&](auto tile, int id, bool vec) {
-        Choice c{d, 0.f, id, vec};
-        const bool quads = vec && !d.up_h;
-        if (direct_plan<decltype(tile)>(c.d, batches, kh, quads, vec && flat, &c.us)) {
-            if (!vec) c.us *= 1.1f;  // four times the load instructions
-            if (best.tile < 0 || c.us < best.us) best = c;
-        }
+// The kernel a convolution runs: a tile of the direct kernel, or the gather core.
+enum ConvRoute { kConvBig, kConvMid, kConvLow, kConvMin, kConvGather };
+using ConvBig = DirectTile<128, 160, 2, 2, 8, 9, 1>;
+using ConvMid = DirectTile<64, 128, 2, 2, 4, 9, 1>;
+using ConvLow = DirectTile<32, 64, 1, 4, 4, 9, 1>;
+using ConvMin = DirectTile<32, 32, 2, 2, 4, 9, 1>;
+struct ConvChoice { ConvRoute route; bool vec, flat; };
+
+// Plans every tile and fills in the plan with the least estimate; the gather
+// core when none takes the shape.
+ConvChoice conv_direct_best(DirectConv &d, int batches, int kh, bool wv, bool flat) {
+    ConvChoice best{kConvGather, false, false};
+    const DirectConv shape = d;
+    float least = 0.f;
+    auto offer = [&](auto tile, ConvRoute route, bool vec) {
+        DirectConv p = shape;
+        float us;
+        if (!direct_plan<decltype(tile)>(p, batches, kh, vec && !p.up_h, vec && flat, &us)) return;
+        if (!vec) us *= 1.1f;  // four times the load instructions
+        if (best.route != kConvGather && us >= least) return;
+        least = us;
+        best = ConvChoice{route, vec, vec && flat};
+        d = p;
     };
     for (bool vec : {true, false}) {
         if (vec && !wv) continue;
-        if (vec || !d.up_h) offer(Big{}, 0, vec);
-        offer(Mid{}, 1, vec);
-        offer(Low{}, 2, vec);
-        offer(Min{}, 3, vec);
+        if (vec || !d.up_h) offer(ConvBig{}, kConvBig, vec);
+        offer(ConvMid{}, kConvMid, vec);
+        offer(ConvLow{}, kConvLow, vec);
+        offer(ConvMin{}, kConvMin, vec);
     }
-    const bool f = best.vec && flat;
-    switch (best.tile) {
-        case 0: conv_direct_launch<Big>(best.d, batches, best.vec, f, s); break;
-        case 1: conv_direct_launch<Mid>(best.d, batches, best.vec, f, s); break;
-        case 2: conv_direct_launch<Low>(best.d, batches, best.vec, f, s); break;
-        case 3: conv_direct_launch<Min>(best.d, batches, best.vec, f, s); break;
-        default: return false;
-    }
-    return true;
+    return best;
 }
 
-// The direct kernel for this convolution, or false when the shape is not one
-// it takes: more than 36 taps, a transposed layer whose kernel is not its
+// The direct kernel's plan for this convolution, or the gather core when the
+// shape is not one it takes: more than 36 taps, a transposed layer whose kernel is not its
 // stride (or padded, or cropped), an image or weight tensor of 1 GiB or more,
 // or a stride so large that no patch fits.
 //
@@ -416,16 +416,16 @@ bool conv_direct_best(const DirectConv &d, int batches, int kh, bool wv, bool fl
 // 90 376 -> 37 us.  By tile: 3x3 512 -> 128 on 64 x 64 27 us with 32 x 64 tiles
 // (40 with 64 x 128, 30 with 32 x 32), 3x3 64 -> 64 on 2 x 128 x 128 12 us with
 // 64 x 128 (18 with 128 x 160, 19 with 32 x 64).
-bool conv_direct(const bf_cuda_conv2d_desc *c, const float *x, const float *w, const float *b,
-                 float *y, hipStream_t s) {
-    DirectConv d{};
+ConvChoice conv_direct(const bf_cuda_conv2d_desc *c, const float *x, const float *w, const float *b,
+                       float *y, DirectConv &d) {
+    constexpr ConvChoice kNone{kConvGather, false, false};
     d.x = x; d.w = w; d.bias = b; d.y = y;
     d.Ci = c->input_channels; d.relu = c->relu;
     d.IH = c->input_height; d.IW = c->input_width;
     const long long hw = (long long)d.IH * d.IW, taps = (long long)c->kernel_height * c->kernel_width;
     const long long columns = c->output_channels * (c->transpose ? taps : 1);
     const long long x_bytes = 4 * hw * d.Ci, w_bytes = 4 * taps * d.Ci * c->output_channels;
-    if (taps > 36 || hw >= 1ll << 28 || x_bytes >= 1ll << 30 || w_bytes >= 1ll << 30) return false;
+    if (taps > 36 || hw >= 1ll << 28 || x_bytes >= 1ll << 30 || w_bytes >= 1ll << 30) return kNone;
     d.columns = (int)columns;
     d.x_bytes = (uint32_t)x_bytes;
     d.w_bytes = (uint32_t)w_bytes;
@@ -434,7 +434,7 @@ bool conv_direct(const bf_cuda_conv2d_desc *c, const float *x, const float *w, c
         if (c->kernel_height != c->stride_height || c->kernel_width != c->stride_width ||
             c->padding_height || c->padding_width ||
             c->output_height != (long long)d.IH * kh || c->output_width != (long long)d.IW * c->kernel_width)
-            return false;
+            return kNone;
         d.up_h = kh; d.up_w = c->kernel_width; d.up_ow = d.IW;
         d.pairs = kh == 2 && d.up_w == 2 && ((uintptr_t)y & 7) == 0;
         d.khw = d.kw = kh = 1;
@@ -454,7 +454,16 @@ bool conv_direct(const bf_cuda_conv2d_desc *c, const float *x, const float *w, c
     }
     const bool wv = aligned16(w) && (c->transpose ? d.columns % 4 == 0 : (long long)d.Ci * d.khw % 4 == 0);
     const bool flat = wv && one && hw % 4 == 0 && aligned16(x);
-    return conv_direct_best(d, c->batches, kh, wv, flat, s);
+    return conv_direct_best(d, c->batches, kh, wv, flat);
+}
+
+void conv_direct_run(const ConvChoice &c, const DirectConv &d, int batches, hipStream_t s) {
+    switch (c.route) {
+        case kConvBig: conv_direct_launch<ConvBig>(d, batches, c.vec, c.flat, s); break;
+        case kConvMid: conv_direct_launch<ConvMid>(d, batches, c.vec, c.flat, s); break;
+        case kConvLow: conv_direct_launch<ConvLow>(d, batches, c.vec, c.flat, s); break;
+        default: conv_direct_launch<ConvMin>(d, batches, c.vec, c.flat, s); break;
+    }
 }
 
 }  // namespace
@@ -489,8 +498,10 @@ extern "C" int bf_cuda_conv2d_f32(const bf_cuda_conv2d_desc *d, const float *inp
     const long long tiles = ((long long)g.M + 127) / 128 * ((Co + 31LL) / 32);
     if (tiles > INT_MAX) return fail(error, cap, "HIP convolution grid is too large");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (conv_direct(d, input, weight, bias, output, s))
-        ;
+    DirectConv direct{};
+    const ConvChoice choice = conv_direct(d, input, weight, bias, output, direct);
+    if (choice.route != kConvGather)
+        conv_direct_run(choice, direct, d->batches, s);
     else if (Co <= 32)
         conv_dispatch_tile<Tile<128, 32, 32, 4, 1>>(g, Co, input, weight, bias, output, d->relu, s);
     else if (Co <= 64)
@@ -526,4 +537,14 @@ extern "C" int bf_cuda_gemm_f32(const float *input, const float *weight, const f
 extern "C" int bfhip_gemm_route(const float *x, const float *w, const float *b, const float *y,
                                 int rows, int in_f, int out_f) {
     return gemm_f32_route(x, w, b, y, rows, in_f, out_f);
+}
+
+extern "C" int bfhip_conv_route(const bf_cuda_conv2d_desc *desc, const float *x, const float *w,
+                                const float *y, unsigned long long *threads) {
+    DirectConv d{};
+    const ConvChoice c = conv_direct(desc, x, w, nullptr, const_cast<float *>(y), d);
+    constexpr int kThreads[] = {ConvBig::kThreads, ConvMid::kThreads, ConvLow::kThreads, ConvMin::kThreads};
+    *threads = c.route == kConvGather ? 0ull
+                                      : (unsigned long long)d.tiles_y * d.tiles_x * d.tiles_c * desc->batches * kThreads[c.route];
+    return c.route;
 }

@@ -332,3 +332,18 @@ def test_gemm_very_many_rows(device):
     bfhip.gemm_f32(x, w, out=out)
     for a in range(0, m, 2 ** 28):
         assert torch.equal(out[a:a + 2 ** 28], x[a:a + 2 ** 28].bfloat16().float() * 0.5), a
+
+
+def test_conv_very_many_pixels(device):
+    """1.25 * 2^30 output pixels: more than a launch of the direct kernel holds.
+    One product per element, so the result is exact."""
+    import bfhip
+    import torch
+    shape = (20, 1, 8192, 8192)
+    x = torch.randn(shape, device=device)
+    w = torch.full((1, 1, 1, 1), 0.5, device=device)
+    out = torch.empty(shape, device=device)
+    print(f"[case] conv 1x1 on {shape}", flush=True)
+    bfhip.conv2d_f32(x, w, out=out)
+    for n in range(shape[0]):
+        assert torch.equal(out[n], x[n].bfloat16().float() * 0.5), n

@@ -46,3 +46,34 @@ def test_gemm_grids_fit_a_launch(n):
 def test_gemm_route_of_very_many_rows():
     """2^30 rows and a few: the thin and 64-row tiles no longer fit."""
     assert gemm_route(2 ** 30 + 77, 1, 1) == 5
+
+
+def conv_route(d, aligned=True):
+    f = bfhip.hip_lib().bfhip_conv_route
+    f.argtypes = [C.c_void_p] * 4 + [C.c_void_p]
+    p, threads = 4096 if aligned else 4100, C.c_ulonglong()
+    return f(C.byref(d), p, p, p, C.byref(threads)), threads.value
+
+
+@pytest.mark.parametrize("ci,co", [(1, 1), (1, 33), (3, 64), (8, 8), (8, 129), (64, 1024)])
+def test_conv_grids_fit_a_launch(ci, co):
+    """Batches of images up to the 2^31 - 1 output pixels a call may have, 1x1,
+    3x3, strided and transposed."""
+    for h, w in ((1, 1), (7, 5), (64, 64), (1024, 1024), (16000, 16000)):
+        for k, s, tr in ((1, 1, 0), (3, 1, 0), (1, 2, 0), (2, 2, 1)):
+            oh, ow = (h * s, w * s) if tr else ((h - 1) // s + 1, (w - 1) // s + 1)
+            for pixels in (10 ** 5, 2 ** 28, 2 ** 29 + 1, 2 ** 30, 2 ** 30 + 2 ** 28, 2 ** 31 - 1):
+                n = max(1, pixels // (oh * ow))
+                if n * oh * ow > 2 ** 31 - 1:
+                    continue
+                d = bfhip.ConvDesc(n, ci, co, h, w, k, k, s, s, 0 if tr else k // 2,
+                                   0 if tr else k // 2, oh, ow, tr, 0)
+                for aligned in (True, False):
+                    assert conv_route(d, aligned)[1] <= LIMIT, (n, h, w, k, s, tr)
+
+
+def test_conv_route_of_very_many_pixels():
+    """1.25 * 2^30 one-channel pixels: more than any direct tile's launch holds
+    (4 to 16 threads a pixel), so the gather core's (2) runs."""
+    d = bfhip.ConvDesc(20, 1, 1, 8192, 8192, 1, 1, 1, 1, 0, 0, 8192, 8192, 0, 0)
+    assert conv_route(d)[0] == 4
