@@ -33,8 +33,6 @@
 
 #include "gemm_core.h"
 
-#include <cmath>
-
 namespace bfhip {
 
 // What one launch needs of the shape.  Columns: output channels, or
@@ -346,7 +344,7 @@ __global__ __launch_bounds__(T::kThreads) void conv_direct_kernel(DirectConv d) 
     }
 }
 
-// Estimated microseconds of a launch with `d`'s plan: the longer of
+// Estimated microseconds of a launch: the longer of
 // - throughput: a CU fetches its workgroups' blocks at about 47 KB/us (fp32
 //   weights and patch: blocks of the 128 x 160, 64 x 64 and 32 x 64 tiles took
 //   3.7, 1.85 and 1.1 us), and each workgroup's first fetch and stores add a
@@ -355,58 +353,73 @@ __global__ __launch_bounds__(T::kThreads) void conv_direct_kernel(DirectConv d) 
 // Against 22 shapes on MI355X it picks the fastest tile or one within 15 % of
 // it (conv 3x3 256 -> 256 on 6 x 32 x 88: 128 x 160 tiles 42 us, estimate 40;
 // 64 x 128 72, 64; 32 x 64 102, 101).
+// fetch_kb: fp32 kilobytes that a workgroup fetches over all its blocks.
 template <class T>
-inline float direct_estimate(const DirectConv &d, int batches) {
+inline float direct_estimate(long long grid, float blocks, float fetch_kb) {
     constexpr size_t kLds = ((size_t)T::kSlots * T::kWRow + T::kUnits + 1) * sizeof(bf16x8);
     constexpr int kPerCu = kLds > 80 * 1024 ? 1 : kLds > 53 * 1024 ? 2 : 4;
     constexpr float kEnds = 2.5f + T::BC * T::BP / 2048.f;
-    const float grid = (float)d.tiles_y * d.tiles_x * d.tiles_c * batches;
-    const float blocks = (float)((d.Ci + 8 * d.O - 1) / (8 * d.O));
-    const float block_kb = 0.032f * d.O * (T::BC * d.khw + d.patch);
-    const float wait = ceilf(grid / (256.f * kPerCu)) * (1.3f * blocks + kEnds);
-    const float fetch = ceilf(grid / 256.f) * (blocks * block_kb / 47.f + 0.8f * kEnds);
+    const float wait = (float)((grid + 256 * kPerCu - 1) / (256 * kPerCu)) * (1.3f * blocks + kEnds);
+    const float fetch = (float)((grid + 255) / 256) * (fetch_kb / 47.f + 0.8f * kEnds);
     return fetch > wait ? fetch : wait;
 }
 
-// Fills in the rectangle, channel block and tile counts of tile T with the
-// least estimate; false when no rectangle's patch fits, an offset could leave
-// 32 bits or the grid is more than a launch holds.  quads: whole quads of slots per block (WV); flat: rectangles
-// of whole pixel quads (XV).
+// The rectangle, channel block and tile counts that tile T gives a layer.
+struct DirectPlan {
+    float us = -1.f;  // estimate, < 0: no plan
+    int TH, TW, O, patch_w, patch, tiles_y, tiles_x;
+};
+
+// Tile T's plan with the least estimate below `limit`; none when no rectangle's
+// patch fits, an offset could leave 32 bits or the grid is more than a launch
+// holds.  quads: whole quads of slots per block (WV); flat: rectangles of whole
+// pixel quads (XV).  This runs on every call, so tiles and rectangles are
+// dropped as soon as a bound of their estimate (the reduction fetched as one
+// block) reaches the limit.  Planned one after the other in full, 3x3 256 -> 256
+// on 6 x 32 x 88 took 2.6 us of host time; now 0.3 (random layers 0.9, now 0.4).
 template <class T>
-inline bool direct_plan(DirectConv &d, int batches, int kh, bool quads, bool flat, float *us) {
+inline DirectPlan direct_plan(const DirectConv &d, int batches, int kh, bool quads, bool flat, float limit) {
     const int octets = (d.Ci + 7) / 8, o_step = quads ? (d.khw % 4 == 0 ? 1 : d.khw % 2 == 0 ? 2 : 4) : 1;
-    const long long wrow = d.up_h ? d.columns : d.khw;
-    DirectConv best = d;
-    *us = -1.f;
-    d.tiles_c = (d.columns + T::BC - 1) / T::BC;
-    for (int th : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 32, 64}) {
+    const int most = T::kSlots / d.khw < octets ? T::kSlots / d.khw : octets;  // octets per block, before rounding
+    const long long wrow = d.up_h ? d.columns : d.khw, hw = (long long)d.IH * d.IW;
+    const long long across = (long long)((d.columns + T::BC - 1) / T::BC) * batches;
+    DirectPlan best;
+    // No rectangle does better than whole tiles of pixels and no patch at all.
+    const float weights_kb = 0.032f * (float)(T::BC * d.khw);
+    const long long pixels = (long long)d.OH * d.OW;
+    if (0.999f * direct_estimate<T>((pixels + T::BP - 1) / T::BP * across, 1.f, weights_kb * (float)octets) >= limit)
+        return best;
+    constexpr int kHeights[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 32, 64};
+#pragma clang loop unroll(full)
+    for (int i = 0; i < 13; ++i) {
+        const int th = kHeights[i];
         if (th > T::BP || (th > d.OH && th > 1)) break;
         // The rectangle's columns, spread evenly over the tiles of a row.
-        int tw = T::BP / th < d.OW ? T::BP / th : d.OW;
-        tw = (d.OW + (d.OW + tw - 1) / tw - 1) / ((d.OW + tw - 1) / tw);
+        const int in_row = (d.OW + T::BP / th - 1) / (T::BP / th);
+        int tw = in_row > 1 ? (d.OW + in_row - 1) / in_row : d.OW;
         if (flat) tw = (tw + 3) / 4 * 4;
-        const long long pw = (long long)(tw - 1) * d.SW + d.kw, patch = pw * ((long long)(th - 1) * d.SH + kh);
-        if (tw * th > T::BP || patch > T::kUnits) continue;
-        int o = (int)(T::kUnits / patch);  // octets per block: what fits, spread evenly over the blocks
-        if (o > T::kSlots / d.khw) o = T::kSlots / d.khw;
-        if (o > octets) o = octets;
+        const long long pw = (long long)(tw - 1) * d.SW + d.kw, area = pw * ((long long)(th - 1) * d.SH + kh);
+        if (tw * th > T::BP || area > T::kUnits) continue;
+        const int ty = (d.OH + th - 1) / th, tx = in_row > 1 ? (d.OW + tw - 1) / tw : 1, patch = (int)area;
+        const long long grid = (long long)ty * tx * across;
+        const float octet_kb = 0.032f * (float)(T::BC * d.khw + patch);
+        if (0.999f * direct_estimate<T>(grid, 1.f, octet_kb * (float)octets) >= limit) continue;
+        int o = T::kUnits / patch;  // octets per block: what fits, spread evenly over the blocks
+        if (o > most) o = most;
         if (o < 1) continue;
         const int nb = (octets + o - 1) / o;
         o = ((octets + nb - 1) / nb + o_step - 1) / o_step * o_step;
         if (o * d.khw > T::kSlots || o * patch > T::kUnits) o -= o_step;
-        if (o < 1 || 32ll * o * d.IH * d.IW >= 1ll << 30 || 32ll * o * wrow >= 1ll << 30) continue;
-        d.TH = th; d.TW = tw; d.O = o; d.patch_w = (int)pw; d.patch = (int)patch;
-        const long long ty = (d.OH + th - 1) / th, tx = (d.OW + tw - 1) / tw;
-        if (!launch_fits(ty * tx * d.tiles_c * batches, T::kThreads)) continue;
-        d.tiles_y = (int)ty; d.tiles_x = (int)tx;
-        const float e = direct_estimate<T>(d, batches);
-        if (*us < 0.f || e < *us) {
-            *us = e;
-            best = d;
+        if (o < 1 || 32 * o * hw >= 1ll << 30 || 32 * o * wrow >= 1ll << 30) continue;
+        if (!launch_fits(grid, T::kThreads)) continue;
+        const float blocks = (float)((octets + o - 1) / o);
+        const float us = direct_estimate<T>(grid, blocks, blocks * (octet_kb * (float)o));
+        if (us < limit) {
+            limit = us;
+            best = DirectPlan{us, th, tw, o, (int)pw, patch, ty, tx};
         }
     }
-    d = best;
-    return *us >= 0.f;
+    return best;
 }
 
 }  // namespace bfhip

@@ -381,18 +381,18 @@ struct ConvChoice { ConvRoute route; bool vec, flat; };
 // Plans every tile and fills in the plan with the least estimate; the gather
 // core when none takes the shape.
 ConvChoice conv_direct_best(DirectConv &d, int batches, int kh, bool wv, bool flat) {
+    DirectPlan plan;
     ConvChoice best{kConvGather, false, false};
-    const DirectConv shape = d;
-    float least = 0.f;
+    float limit = INFINITY;
     auto offer = [&](auto tile, ConvRoute route, bool vec) {
-        DirectConv p = shape;
-        float us;
-        if (!direct_plan<decltype(tile)>(p, batches, kh, vec && !p.up_h, vec && flat, &us)) return;
-        if (!vec) us *= 1.1f;  // four times the load instructions
-        if (best.route != kConvGather && us >= least) return;
-        least = us;
+        using T = decltype(tile);
+        const float scale = vec ? 1.f : 1.1f;  // scalar: four times the load instructions
+        const DirectPlan p = direct_plan<T>(d, batches, kh, vec && !d.up_h, vec && flat, limit / scale);
+        if (p.us < 0.f || scale * p.us >= limit) return;
+        limit = scale * p.us;
+        plan = p;
         best = ConvChoice{route, vec, vec && flat};
-        d = p;
+        d.tiles_c = (d.columns + T::BC - 1) / T::BC;
     };
     for (bool vec : {true, false}) {
         if (vec && !wv) continue;
@@ -401,6 +401,8 @@ ConvChoice conv_direct_best(DirectConv &d, int batches, int kh, bool wv, bool fl
         offer(ConvLow{}, kConvLow, vec);
         offer(ConvMin{}, kConvMin, vec);
     }
+    d.TH = plan.TH; d.TW = plan.TW; d.O = plan.O; d.patch_w = plan.patch_w; d.patch = plan.patch;
+    d.tiles_y = plan.tiles_y; d.tiles_x = plan.tiles_x;
     return best;
 }
 
