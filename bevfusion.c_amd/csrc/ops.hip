@@ -52,10 +52,6 @@ constexpr int kPanelWaves = 8;
 constexpr int kPanelThreads = kPanelWaves * kWave;
 constexpr int kPanelRows = 16 * kPanelWaves;
 constexpr int kPanelMaxFrags = 9;  // column blocks per half: N <= 288
-// Below this the panels leave most CUs idle (K = 96, N = 288, panel against
-// tiled core: M = 500 6.1 vs 3.1 us, 3000 6.5 vs 4.6, 9000 8.2 vs 7.5, 11264
-// 8.4 vs 8.8).
-constexpr int kPanelMinRows = 10240;
 
 inline int panel_cols(int N) { return 16 * (((N + 15) / 16 + 1) / 2); }  // per column half
 inline size_t panel_lds_bytes(int N, int ks) { return (size_t)panel_cols(N) * 8 * ks * 16; }
@@ -140,9 +136,9 @@ __global__ __launch_bounds__(kPanelThreads) void gemm_f32_panel_kernel(
 }
 
 // Whether the panel kernel takes the shape.
-bool gemm_f32_panel_takes(const float *x, const float *w, const float *b, const float *y, int M,
-                          int K, int N) {
-    return M >= kPanelMinRows && K <= 128 && !(K & 3) && !(N & 3) && N > 144 &&
+bool gemm_f32_panel_takes(const float *x, const float *w, const float *b, const float *y, int K,
+                          int N) {
+    return K <= 128 && !(K & 3) && !(N & 3) && N > 144 &&
            N <= 2 * 16 * kPanelMaxFrags && (long long)N * K * 4 < (1ll << 31) && aligned16(x) &&
            aligned16(w) && aligned16(y) && (!b || aligned16(b)) &&
            panel_lds_bytes(N, (K + 31) / 32) <= 65536;
@@ -264,53 +260,95 @@ void gemm_f32_thin_launch(const float *x, const float *w, const float *b, float 
                        0, s, x, w, b, y, M, K, N, tiles_n, relu);
 }
 
-// The kernel with the least estimated time (microseconds) of those whose grid a
-// launch holds: a CU fetches its workgroups' operands at about 60 KB/us (33 for
-// the thin kernel's scattered rows), each workgroup and launch adds a constant,
-// and a k-block takes at least its fetch latency.  Fitted to 29 shapes on
-// MI355X; the choice is within 7 % of the fastest at every one of them.  Against
-// the 128 x 128 x 32, 32 x 144 and 128 x 32 tiles used before: 4224 x 384 ->
-// 1536 33.1 -> 18.8 us (265 TFLOP/s; 128 x 128 tiles, 64-deep blocks, eight
-// waves), 300 x 1024 -> 1024 11.1 (32 x 32 tiles, 128-deep; 18 with 64 x 64),
-// 16896 x 192 -> 768 28.9 (32 with 64 x 64 tiles).  From some 10^9 rows only the
-// four-wave 128 x 128 tile has few enough threads; kGemmNone: none has.
-enum GemmRoute { kGemmNone = -1, kGemm128, kGemm64, kGemm32, kGemmThinSplit, kGemmThinRows, kGemmWide, kGemmPanel };
+enum GemmRoute {
+    kGemmNone = -1, kGemm128, kGemm64, kGemm32, kGemmThinSplit, kGemmThinRows, kGemmWide, kGemmPanel, kGemm128x32, kGemm128x64
+};
 using Gemm128 = Tile<128, 128, 64, 2, 4>;
 using Gemm64 = Tile<64, 64, 64, 2, 2>;
 using Gemm32 = Tile<32, 32, 128, 2, 2>;
+using Gemm128x32 = Tile<128, 32, 32, 4, 1>;
+using Gemm128x64 = Tile<128, 64, 32, 4, 1>;
 using GemmWide = Tile<128, 128, 32, 2, 2>;
 
-GemmRoute gemm_route(int M, int K, int N) {
-    auto ceil_div = [](long long a, long long b) { return (a + b - 1) / b; };
-    auto tiles = [&](int bm, int bn) { return ceil_div(M, bm) * ceil_div(N, bn); };
-    auto tiled = [&](int bm, int bn, int bk, int per_cu, float launch, float each, float block) {
-        const float g = (float)tiles(bm, bn), kb = (bm + bn) * (float)K * 0.004f;
-        const float wait = ceilf(g / (256.f * per_cu)) * (float)ceil_div(K, bk) * block;
-        const float fetch = ceilf(g / 256.f) * (kb / 60.f + each);
-        return launch + (fetch > wait ? fetch : wait);
-    };
-    auto thin = [&](int wm, int kw, float launch, int per_cu) {
-        const float g = (float)tiles(16 * wm, 16), kb = (16 * wm + 16) * (float)K * 0.004f;
-        const float wait = ceilf(g / (256.f * per_cu)) * (float)ceil_div(K, 32 * kw) * 0.8f;
-        const float fetch = g / 256.f * (kb / 33.f + 0.25f);
-        return launch + (fetch > wait ? fetch : wait);
-    };
+// What a launch takes, in microseconds: launch + sqrt(fetch^2 + wait^2) + store
+// per megabyte of Y, with
+//   fetch: rounds of one workgroup per CU, each its operands' KB / rate + each,
+//          but no less than all workgroups' KB at `flow` per CU;
+//   wait:  rounds of per_cu workgroups per CU, each its k-blocks x block.
+struct GemmCost {
+    GemmRoute route;
+    int rows, cols, depth, per_cu, threads;  // the workgroup's tile and its k-block
+    float launch, each, rate, block, store, flow;
+    constexpr float us(long long grid, float blocks, float kb, float mb) const {
+        const float alone = (float)((grid + 255) / 256) * (kb / rate + each), all = (float)grid * kb / (256.f * flow);
+        const float fetch = alone > all ? alone : all;
+        const float wait = (float)((grid + 256 * per_cu - 1) / (256 * per_cu)) * blocks * block;
+        return launch + sqrtf(fetch * fetch + wait * wait) + store * mb;
+    }
+};
+// Fitted on MI355X to the times of every kernel at 3989 shapes (rows to
+// 400 000, K and N to 8192, most of them spread over the logarithm of sizes up
+// to 2.5 G products; a third with K <= 128), apart for operands that are loaded
+// as floats (first) and as float4.
+constexpr GemmCost kGemmCosts[2][7] = {
+    {{kGemm128, 128, 128, 64, 2, Gemm128::kThreads, 2.68f, 1.28f, 20.5f, 2.37f, 0.419f, 19.6f},
+     {kGemm64, 64, 64, 64, 4, Gemm64::kThreads, 2.56f, 0.521f, 19.4f, 1.57f, 0.369f, 18.6f},
+     {kGemm32, 32, 32, 128, 4, Gemm32::kThreads, 2.35f, 0.336f, 9.5f, 1.5f, 0.361f, 8.82f},
+     {kGemmThinSplit, 16, 16, 256, 4, 8 * kWave, 2.21f, 0.165f, 16.9f, 1.03f, 1.44f, 13.f},
+     {kGemmThinRows, 64, 16, 32, 8, 4 * kWave, 2.41f, 0.283f, 64.2f, 0.801f, 0.393f, 9.44f},
+     {kGemm128x32, 128, 32, 32, 4, Gemm128x32::kThreads, 2.64f, 0.f, 15.6f, 1.21f, 0.447f, 80.f},
+     {kGemm128x64, 128, 64, 32, 4, Gemm128x64::kThreads, 2.73f, 0.f, 17.4f, 1.45f, 0.432f, 21.6f}},
+    {{kGemm128, 128, 128, 64, 2, Gemm128::kThreads, 3.67f, 0.502f, 85.5f, 1.05f, 0.229f, 60.6f},
+     {kGemm64, 64, 64, 64, 4, Gemm64::kThreads, 2.87f, 0.473f, 158.f, 0.924f, 0.192f, 70.9f},
+     {kGemm32, 32, 32, 128, 4, Gemm32::kThreads, 2.64f, 0.398f, 1000.f, 0.881f, 0.253f, 77.1f},
+     {kGemmThinSplit, 16, 16, 256, 4, 8 * kWave, 2.32f, 0.326f, 125.f, 0.453f, 0.71f, 40.8f},
+     {kGemmThinRows, 64, 16, 32, 8, 4 * kWave, 2.66f, 0.183f, 1000.f, 0.264f, 0.306f, 35.2f},
+     {kGemm128x32, 128, 32, 32, 4, Gemm128x32::kThreads, 2.9f, 0.348f, 1000.f, 0.679f, 0.225f, 65.1f},
+     {kGemm128x64, 128, 64, 32, 4, Gemm128x64::kThreads, 3.f, 0.522f, 173.f, 0.781f, 0.215f, 69.1f}}};
+constexpr GemmCost kPanelCost = {kGemmPanel, kPanelRows, 0, 32, 2, kPanelThreads, 2.89f, 0.f, 55.1f, 0.0696f, 0.202f, 10000.f};
+
+// The kernel with the least estimated time of those whose grid a launch holds.
+// At those shapes the choice costs 0.9 % over the fastest kernel in the mean. At
+// 14 of them it is more than 4 % slower than the tile that N alone used to name
+// (128 x 32 to N = 32, 128 x 64 to 64, the panels or 32 x 144 from 145 to 288,
+// four waves on 128 x 128 elsewhere): at most 12 % up to 2.5 G products, 36 % for
+// 10 882 x 129 -> 3104.  With estimates that left out the stores and took one set
+// of rates for both load widths, and the panels only from 10 240 rows on, it
+// cost 4.8 %: 17 406 x 14 -> 13 6.3 us (now 3.9; the tile by N 4.6), 9000 x 8 ->
+// 200 7.7 (panels: 4.5), 2865 x 337 -> 277 41 (17; 26).  Others: 4224 x 384 ->
+// 1536 33.1 -> 18.8 us (265 TFLOP/s; 128 x 128, 64-deep, eight waves), 300 x 1024
+// -> 1024 11.1 (32 x 32; 18 with 64 x 64), 35 x 2590 -> 265 402 -> 27.  From some
+// 10^9 rows on only four-wave tiles of 128 rows have few enough threads;
+// kGemmNone: no kernel has.
+template <bool VEC>
+GemmRoute gemm_route(int M, int K, int N, bool panel) {
+    const auto ceil_div = [](long long a, long long b) { return (a + b - 1) / b; };
+    const float mb = (float)M * (float)N * 4e-6f;
     float best = INFINITY;
     GemmRoute pick = kGemmNone;
-    auto offer = [&](GemmRoute id, int bm, int bn, int threads, float us) {
-        if (us < best && launch_fits(tiles(bm, bn), threads)) {
+    const auto offer = [&](const GemmCost &c, long long grid, float blocks, float kb) {
+        const float us = c.us(grid, blocks, kb, mb);
+        if (us < best && launch_fits(grid, c.threads)) {
             best = us;
-            pick = id;
+            pick = c.route;
         }
     };
-    offer(kGemm128, 128, 128, Gemm128::kThreads, tiled(128, 128, 64, 2, 4.5f, 1.3f, 1.6f));
-    offer(kGemm64, 64, 64, Gemm64::kThreads, tiled(64, 64, 64, 4, 2.7f, 0.5f, 1.05f));
-    offer(kGemm32, 32, 32, Gemm32::kThreads, tiled(32, 32, 128, 4, 2.1f, 0.25f, 1.0f));
-    if (K <= 1 << 20 && tiles(16, 16) < 1000000000) {
-        offer(kGemmThinSplit, 16, 16, 8 * kWave, thin(1, 8, 2.1f, 4));
-        offer(kGemmThinRows, 64, 16, 4 * kWave, thin(4, 1, 2.6f, 8));
+#pragma clang loop unroll(full)
+    for (int i = 0; i < 7; ++i) {
+        const GemmCost &c = kGemmCosts[VEC][i];
+        // The thin kernel's fragment offsets are 32-bit; past N = 32 the 128 x 64
+        // tile reads X half as often.
+        if ((c.route == kGemmThinSplit || c.route == kGemmThinRows) && K > 1 << 20) continue;
+        if (c.route == kGemm128x32 && N > 32) continue;
+        offer(c, ceil_div(M, c.rows) * ceil_div(N, c.cols), (float)ceil_div(K, c.depth),
+              (float)(c.rows + c.cols) * (float)K * 0.004f);
     }
-    if (pick == kGemmNone && launch_fits(tiles(128, 128), GemmWide::kThreads)) pick = kGemmWide;
+    if (panel) {
+        const int cols = panel_cols(N);
+        offer(kPanelCost, 2 * ceil_div(M, kPanelRows), (float)(ceil_div(K, 32) * (cols / 16)),
+              (float)(kPanelRows + cols) * (float)K * 0.004f);
+    }
+    if (pick == kGemmNone && launch_fits(ceil_div(M, 128) * ceil_div(N, 128), GemmWide::kThreads)) pick = kGemmWide;
     return pick;
 }
 
@@ -323,13 +361,18 @@ void gemm_f32_dispatch(GemmRoute route, const float *x, const float *w, const fl
         case kGemm32: gemm_f32_launch<Gemm32, VEC>(x, w, b, y, M, K, N, relu, s); break;
         case kGemmThinSplit: gemm_f32_thin_launch<1, 8, VEC>(x, w, b, y, M, K, N, relu, s); break;
         case kGemmThinRows: gemm_f32_thin_launch<4, 1, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        case kGemm128x32: gemm_f32_launch<Gemm128x32, VEC>(x, w, b, y, M, K, N, relu, s); break;
+        case kGemm128x64: gemm_f32_launch<Gemm128x64, VEC>(x, w, b, y, M, K, N, relu, s); break;
         default: gemm_f32_launch<GemmWide, VEC>(x, w, b, y, M, K, N, relu, s); break;
     }
 }
 
+bool gemm_f32_vec(const float *x, const float *w, int K) { return (K & 3) == 0 && aligned16(x) && aligned16(w); }
+
 GemmRoute gemm_f32_route(const float *x, const float *w, const float *b, const float *y, int M,
                          int K, int N) {
-    return gemm_f32_panel_takes(x, w, b, y, M, K, N) ? kGemmPanel : gemm_route(M, K, N);
+    if (!gemm_f32_vec(x, w, K)) return gemm_route<false>(M, K, N, false);
+    return gemm_route<true>(M, K, N, gemm_f32_panel_takes(x, w, b, y, K, N));
 }
 
 template <class T>
@@ -529,7 +572,7 @@ extern "C" int bf_cuda_gemm_f32(const float *input, const float *weight, const f
     if (route == kGemmNone) return fail(error, cap, "HIP GEMM is too large");
     if (route == kGemmPanel)  // short reduction: one pass per row panel
         gemm_f32_panel(input, weight, bias, output, rows, in_f, out_f, relu, s);
-    else if ((in_f & 3) == 0 && aligned16(input) && aligned16(weight))
+    else if (gemm_f32_vec(input, weight, in_f))
         gemm_f32_dispatch<true>(route, input, weight, bias, output, rows, in_f, out_f, relu, s);
     else
         gemm_f32_dispatch<false>(route, input, weight, bias, output, rows, in_f, out_f, relu, s);

@@ -178,13 +178,22 @@ def test_repeat_is_bit_exact(device):
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+def _gemm_route(*args):
+    """GemmRoute (ops.hip) of a call: asserted, so that a case keeps running the
+    kernel it is there for."""
+    from test_launch_limits import gemm_route
+    return gemm_route(*args)
+
+
 # (rows, in, out, relu, bias, inject Inf/NaN): shapes the short-reduction
-# panel kernel takes (K <= 128, K % 4 == 0, 144 < N <= 288, N % 4 == 0):
-# ragged row panels, N not a multiple of 16, K not a multiple of 8 or 32,
-# one to four 32-deep k-steps, ReLU, no bias, and Inf/NaN operands.
-PANEL_CASES = [(1001, 100, 148, True, True, False), (64, 4, 160, False, False, False),
-               (5, 128, 200, False, True, False), (130, 32, 288, True, True, True),
-               (11264, 96, 288, False, True, False), (65, 60, 252, False, True, False)]
+# panel kernel is chosen for (K <= 128, K % 4 == 0, 144 < N <= 288, N % 4 == 0):
+# ragged row panels (1, 7, 63 and 65 rows in the last), N not a multiple of 16,
+# K not a multiple of 8 or 32, one to four 32-deep k-steps, ReLU, no bias, and
+# Inf/NaN operands.
+PANEL_CASES = [(10241, 100, 148, True, True, False), (4039, 4, 160, False, False, False),
+               (9023, 128, 200, False, True, False), (10305, 32, 288, True, True, True),
+               (11264, 96, 288, False, True, False), (8385, 60, 252, False, True, False),
+               (12353, 124, 244, True, False, True), (4161, 36, 204, False, False, True)]
 
 
 @pytest.mark.parametrize("case", PANEL_CASES)
@@ -199,6 +208,7 @@ def test_gemm_panel_equals_tiled_core(device, case):
     m, k, n, relu, with_bias, special = case
     print(f"[case] panel gemm {m}x{k}->{n} relu={relu} bias={with_bias} special={special}",
           flush=True)
+    assert _gemm_route(m, k, n) == 6
     rng = np.random.default_rng(m + 3 * k + 7 * n)
     x = rng.standard_normal((m, k)).astype(np.float32)
     w = (rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32)
@@ -211,6 +221,7 @@ def test_gemm_panel_equals_tiled_core(device, case):
     panel = bfhip.gemm_f32(xt, wt, bt, relu=relu)
     buf = torch.empty(m * n + 1, device=device)
     tiled_out = buf[1:].view(m, n)
+    assert bfhip.hip_lib().bfhip_gemm_route(4096, 4096, None, 4100, m, k, n) not in (3, 6)
     bfhip.gemm_f32(xt, wt, bt, relu=relu, out=tiled_out)
     torch.cuda.synchronize()
     a, t = panel.cpu().numpy(), tiled_out.cpu().numpy()
@@ -294,6 +305,26 @@ GEMM_EDGE_CASES = [(1, 1, 1, True, True, False), (15, 31, 17, False, True, False
                    (4097, 7, 3, True, False, False), (300, 512, 513, False, True, False),
                    (999, 130, 1001, False, True, True), (6001, 100, 290, True, True, False),
                    (4225, 200, 1540, False, True, False)]
+
+
+# The same with the kernel that is to run: each at the edges of its tile and
+# k-block, loads of four floats and of one, the PANEL_CASES shapes of few rows.
+GEMM_ROUTE_CASES = [(0, (4225, 388, 1540, True, True, False)), (0, (16753, 79, 79, False, True, True)),
+                    (1, (6001, 100, 290, True, True, False)), (1, (2865, 337, 277, False, True, True)),
+                    (2, (300, 1028, 1021, False, True, False)), (2, (500, 259, 401, True, False, True)),
+                    (3, (201, 260, 255, True, True, True)), (3, (6, 2387, 5, False, True, False)),
+                    (3, (64, 4, 160, False, False, False)), (3, (5, 128, 200, False, True, False)),
+                    (3, (130, 32, 288, True, True, True)), (3, (65, 60, 252, False, True, False)),
+                    (4, (17406, 14, 13, True, True, False)), (4, (40190, 142, 1, False, True, True)),
+                    (4, (2500, 8, 161, False, False, True)), (2, (1001, 100, 148, True, True, False)),
+                    (7, (60715, 64, 12, True, True, True)), (7, (91847, 41, 9, False, True, False)),
+                    (8, (82455, 4, 57, True, True, True)), (8, (62014, 31, 57, False, False, False))]
+
+
+@pytest.mark.parametrize("route,case", GEMM_ROUTE_CASES)
+def test_gemm_each_kernel(device, route, case):
+    assert _gemm_route(*case[:3]) == route
+    test_gemm_edges(device, case)
 
 
 @pytest.mark.parametrize("case", GEMM_EDGE_CASES)

@@ -12,7 +12,8 @@ import bfhip
 LIMIT = 2 ** 32 - 1
 # GemmRoute of ops.hip: rows x columns of a workgroup's tile, threads.
 GEMM_TILES = {0: (128, 128, 512), 1: (64, 64, 256), 2: (32, 32, 256), 3: (16, 16, 512),
-              4: (64, 16, 256), 5: (128, 128, 256), 6: (128, 1 << 30, 512)}
+              4: (64, 16, 256), 5: (128, 128, 256), 6: (128, 1 << 30, 512), 7: (128, 32, 256),
+              8: (128, 64, 256)}
 
 
 def _threads(m, n, tile):
@@ -44,8 +45,33 @@ def test_gemm_grids_fit_a_launch(n):
 
 
 def test_gemm_route_of_very_many_rows():
-    """2^30 rows and a few: the thin and 64-row tiles no longer fit."""
-    assert gemm_route(2 ** 30 + 77, 1, 1) == 5
+    """2^30 rows and a few: only four-wave tiles of 128 rows still fit."""
+    assert gemm_route(2 ** 30 + 77, 1, 1) in (5, 7, 8)
+
+
+# Microseconds on MI355X per kernel (GemmRoute), HIP-graph replays, aligned operands.
+GEMM_TIMES = {
+    (200, 128, 256): {0: 6.7, 1: 5.0, 2: 3.7, 3: 3.5, 4: 4.7, 6: 6.9, 7: 5.7, 8: 6.3},
+    (11264, 96, 288): {0: 10.6, 1: 9.4, 2: 12.4, 3: 37.8, 4: 22.4, 6: 8.4, 7: 9.0, 8: 8.6},
+    (4224, 384, 1536): {0: 21.2, 1: 26.0, 2: 41.4, 3: 167.4, 4: 135.7, 7: 30.6, 8: 23.8},
+    (40190, 142, 1): {0: 24.8, 1: 18.6, 2: 25.7, 3: 12.9, 4: 12.9, 7: 16.2, 8: 17.2},
+    (2865, 337, 277): {0: 29.1, 1: 17.3, 2: 41.0, 3: 45.6, 4: 54.9, 7: 23.3, 8: 24.6},
+    (16753, 79, 79): {0: 13.5, 1: 15.9, 2: 20.3, 3: 23.1, 4: 19.6, 7: 14.0, 8: 16.8},
+    (17406, 14, 13): {0: 7.4, 1: 5.9, 2: 6.3, 3: 6.1, 4: 3.9, 7: 4.6, 8: 5.5},
+    (26803, 2, 9): {0: 6.8, 1: 5.3, 2: 5.5, 3: 7.8, 4: 3.8, 7: 4.4, 8: 5.3},
+    (4988, 8, 180): {0: 6.1, 1: 4.7, 2: 5.3, 3: 10.7, 4: 4.5, 6: 4.3, 7: 4.6, 8: 4.8},
+    (8030, 20, 168): {0: 6.5, 1: 5.3, 2: 7.0, 3: 14.7, 4: 5.3, 6: 4.4, 7: 5.1, 8: 5.1},
+    (60714, 64, 12): {0: 7.5, 1: 6.1, 2: 7.5, 3: 11.7, 4: 6.3, 7: 5.3, 8: 6.0},
+    (82454, 4, 56): {0: 12.3, 1: 9.8, 2: 17.3, 3: 46.6, 4: 12.3, 7: 9.2, 8: 8.5},
+    (300, 1024, 1024): {0: 22.8, 1: 18.3, 2: 12.0, 3: 22.2, 4: 31.3, 7: 25.0, 8: 26.7},
+    (16896, 192, 768): {0: 25.3, 1: 26.1, 2: 51.4, 3: 197.1, 4: 138.8, 7: 29.7, 8: 25.0},
+}
+
+
+@pytest.mark.parametrize("shape", sorted(GEMM_TIMES))
+def test_gemm_choice_is_near_the_fastest(shape):
+    times = GEMM_TIMES[shape]
+    assert times[gemm_route(*shape)] <= 1.1 * min(times.values())
 
 
 def conv_route(d, aligned=True):
