@@ -33,6 +33,8 @@
 
 #include "gemm_core.h"
 
+#include <cmath>
+
 namespace bfhip {
 
 // What one launch needs of the shape.  Columns: output channels, or
@@ -344,24 +346,22 @@ __global__ __launch_bounds__(T::kThreads) void conv_direct_kernel(DirectConv d) 
     }
 }
 
-// Estimated microseconds of a launch: the longer of
-// - throughput: a CU fetches its workgroups' blocks at about 47 KB/us (fp32
-//   weights and patch: blocks of the 128 x 160, 64 x 64 and 32 x 64 tiles took
-//   3.7, 1.85 and 1.1 us), and each workgroup's first fetch and stores add a
-//   time that grows with its tile;
-// - latency: a block takes at least 1.3 us (fetch round trip, two barriers).
-// Against 22 shapes on MI355X it picks the fastest tile or one within 15 % of
-// it (conv 3x3 256 -> 256 on 6 x 32 x 88: 128 x 160 tiles 42 us, estimate 40;
-// 64 x 128 72, 64; 32 x 64 102, 101).
-// fetch_kb: fp32 kilobytes that a workgroup fetches over all its blocks.
+// What a launch of the direct kernel takes, in microseconds: base + sqrt(fetch^2
+// + wait^2), base being its launch and its stores, with
+//   fetch: rounds of one workgroup per CU, each the fp32 kilobytes that it
+//          fetches over all its blocks / rate + ends (first fetch, stores);
+//   wait:  rounds of as many workgroups as fit a CU's LDS, each its blocks x
+//          block (fetch round trip, two barriers) + ends.
+struct DirectCost {
+    float base, ends, rate, block;
+};
 template <class T>
-inline float direct_estimate(long long grid, float blocks, float fetch_kb) {
+inline float direct_estimate(const DirectCost &c, long long grid, float blocks, float fetch_kb) {
     constexpr size_t kLds = ((size_t)T::kSlots * T::kWRow + T::kUnits + 1) * sizeof(bf16x8);
-    constexpr int kPerCu = kLds > 80 * 1024 ? 1 : kLds > 53 * 1024 ? 2 : 4;
-    constexpr float kEnds = 2.5f + T::BC * T::BP / 2048.f;
-    const float wait = (float)((grid + 256 * kPerCu - 1) / (256 * kPerCu)) * (1.3f * blocks + kEnds);
-    const float fetch = (float)((grid + 255) / 256) * (fetch_kb / 47.f + 0.8f * kEnds);
-    return fetch > wait ? fetch : wait;
+    constexpr int kPerCu = kLds > 80 * 1024 ? 1 : kLds > 48 * 1024 ? 2 : 4;
+    const float fetch = (float)((grid + 255) / 256) * (fetch_kb / c.rate + c.ends);
+    const float wait = (float)((grid + 256 * kPerCu - 1) / (256 * kPerCu)) * (c.block * blocks + c.ends);
+    return c.base + sqrtf(fetch * fetch + wait * wait);
 }
 
 // The rectangle, channel block and tile counts that tile T gives a layer.
@@ -378,7 +378,8 @@ struct DirectPlan {
 // block) reaches the limit.  Planned one after the other in full, 3x3 256 -> 256
 // on 6 x 32 x 88 took 2.6 us of host time; now 0.3 (random layers 0.9, now 0.4).
 template <class T>
-inline DirectPlan direct_plan(const DirectConv &d, int batches, int kh, bool quads, bool flat, float limit) {
+inline DirectPlan direct_plan(const DirectConv &d, int batches, int kh, bool quads, bool flat, const DirectCost &c,
+                              float limit) {
     const int octets = (d.Ci + 7) / 8, o_step = quads ? (d.khw % 4 == 0 ? 1 : d.khw % 2 == 0 ? 2 : 4) : 1;
     const int most = T::kSlots / d.khw < octets ? T::kSlots / d.khw : octets;  // octets per block, before rounding
     const long long wrow = d.up_h ? d.columns : d.khw, hw = (long long)d.IH * d.IW;
@@ -387,7 +388,7 @@ inline DirectPlan direct_plan(const DirectConv &d, int batches, int kh, bool qua
     // No rectangle does better than whole tiles of pixels and no patch at all.
     const float weights_kb = 0.032f * (float)(T::BC * d.khw);
     const long long pixels = (long long)d.OH * d.OW;
-    if (0.999f * direct_estimate<T>((pixels + T::BP - 1) / T::BP * across, 1.f, weights_kb * (float)octets) >= limit)
+    if (0.999f * direct_estimate<T>(c, (pixels + T::BP - 1) / T::BP * across, 1.f, weights_kb * (float)octets) >= limit)
         return best;
     constexpr int kHeights[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 32, 64};
 #pragma clang loop unroll(full)
@@ -403,7 +404,7 @@ inline DirectPlan direct_plan(const DirectConv &d, int batches, int kh, bool qua
         const int ty = (d.OH + th - 1) / th, tx = in_row > 1 ? (d.OW + tw - 1) / tw : 1, patch = (int)area;
         const long long grid = (long long)ty * tx * across;
         const float octet_kb = 0.032f * (float)(T::BC * d.khw + patch);
-        if (0.999f * direct_estimate<T>(grid, 1.f, octet_kb * (float)octets) >= limit) continue;
+        if (0.999f * direct_estimate<T>(c, grid, 1.f, octet_kb * (float)octets) >= limit) continue;
         int o = T::kUnits / patch;  // octets per block: what fits, spread evenly over the blocks
         if (o > most) o = most;
         if (o < 1) continue;
@@ -413,7 +414,7 @@ inline DirectPlan direct_plan(const DirectConv &d, int batches, int kh, bool qua
         if (o < 1 || 32 * o * hw >= 1ll << 30 || 32 * o * wrow >= 1ll << 30) continue;
         if (!launch_fits(grid, T::kThreads)) continue;
         const float blocks = (float)((octets + o - 1) / o);
-        const float us = direct_estimate<T>(grid, blocks, blocks * (octet_kb * (float)o));
+        const float us = direct_estimate<T>(c, grid, blocks, blocks * (octet_kb * (float)o));
         if (us < limit) {
             limit = us;
             best = DirectPlan{us, th, tw, o, (int)pw, patch, ty, tx};

@@ -43,7 +43,8 @@ extern "C" void bfhip_lidar_offset_limit(bf_cuda_lidar_backbone *backbone, unsig
 extern "C" int bfhip_gemm_route(const float *x, const float *w, const float *b, const float *y,
                                 int rows, int in_f, int out_f);
 
-// For tests: the kernel that bf_cuda_conv2d_f32 runs (ConvRoute in ops.hip) and
-// the threads of its launch (0 for the gather core).
+// For tests: the kernel that bf_cuda_conv2d_f32 runs (ConvRoute in ops.hip, plus
+// 8 where it loads weights as float4 and 16 where the patch too) and the
+// threads of its launch (0 for the gather core).
 extern "C" int bfhip_conv_route(const bf_cuda_conv2d_desc *desc, const float *x, const float *w,
                                 const float *y, unsigned long long *threads);

@@ -421,18 +421,53 @@ using ConvLow = DirectTile<32, 64, 1, 4, 4, 9, 1>;
 using ConvMin = DirectTile<32, 32, 2, 2, 4, 9, 1>;
 struct ConvChoice { ConvRoute route; bool vec, flat; };
 
-// Plans every tile and fills in the plan with the least estimate; the gather
-// core when none takes the shape.
-ConvChoice conv_direct_best(DirectConv &d, int batches, int kh, bool wv, bool flat) {
+// Costs fitted on MI355X to the times of every tile and of the gather core at
+// 3799 layers (draws of up to 20 GFLOP, two fifths of them with at most 64
+// channels, an eighth with up to 2000 small images), in the terms of DirectCost;
+// store: per megabyte of output, of plain and of transposed layers.
+struct ConvCost {
+    float launch, ends, rate, block, store, store_up;
+    float base(float mb, bool up) const { return launch + (up ? store_up : store) * mb; }
+};
+constexpr ConvCost kDirectCosts[2][4] = {  // single floats, float4
+    {{3.33f, 3.8f, 41.7f, 0.f, 0.678f, 1.5f},
+     {3.82f, 2.53f, 31.2f, 0.f, 0.358f, 0.624f},
+     {3.06f, 1.61f, 42.4f, 0.901f, 0.285f, 0.0485f},
+     {3.05f, 1.41f, 40.5f, 0.829f, 0.454f, 0.f}},
+    {{4.35f, 3.15f, 46.6f, 0.f, 0.667f, 0.644f},
+     {4.99f, 1.68f, 41.1f, 0.f, 0.422f, 0.379f},
+     {3.27f, 1.38f, 48.1f, 0.775f, 0.603f, 0.143f},
+     {3.16f, 1.31f, 46.7f, 0.624f, 1.f, 0.f}}};
+// The gather core with 32, 64 and 128 output channels per tile: ends and rate
+// of a tile's operands as fp32, block per 32-deep k-step (times store_up where
+// transposed).
+constexpr ConvCost kGatherCosts[3] = {
+    {4.31f, 0.651f, 8.87f, 2.78f, 0.155f, 2.22f},
+    {5.89f, 1.43f, 11.1f, 2.62f, 0.0767f, 3.03f},
+    {13.4f, 0.f, 13.5f, 3.42f, 0.251f, 2.4f}};
+
+float conv_gather_estimate(const ConvGeom &g, int Co, float mb) {
+    const int id = Co <= 32 ? 0 : Co <= 64 ? 1 : 2, cols = 32 << id, per_cu = id < 2 ? 4 : 2;
+    const ConvCost &c = kGatherCosts[id];
+    const long long grid = ((long long)g.M + 127) / 128 * ((Co + cols - 1) / cols);
+    const float kb = (float)(128 + cols) * (float)g.K * 0.004f, steps = (float)((g.K + 31) / 32);
+    const float fetch = (float)((grid + 255) / 256) * (kb / c.rate + c.ends);
+    const float wait = (float)((grid + 256 * per_cu - 1) / (256 * per_cu)) * steps * c.block * (g.transpose ? c.store_up : 1.f);
+    return c.launch + sqrtf(fetch * fetch + wait * wait) + c.store * mb;
+}
+
+// Plans every tile and fills in the plan with the least estimate below the
+// gather core's, `limit`; the gather core when there is none.
+ConvChoice conv_direct_best(DirectConv &d, int batches, int kh, bool wv, bool flat, float mb, float limit) {
     DirectPlan plan;
     ConvChoice best{kConvGather, false, false};
-    float limit = INFINITY;
     auto offer = [&](auto tile, ConvRoute route, bool vec) {
         using T = decltype(tile);
-        const float scale = vec ? 1.f : 1.1f;  // scalar: four times the load instructions
-        const DirectPlan p = direct_plan<T>(d, batches, kh, vec && !d.up_h, vec && flat, limit / scale);
-        if (p.us < 0.f || scale * p.us >= limit) return;
-        limit = scale * p.us;
+        const ConvCost &c = kDirectCosts[vec][route];
+        const DirectPlan p = direct_plan<T>(d, batches, kh, vec && !d.up_h, vec && flat,
+                                            DirectCost{c.base(mb, d.up_h), c.ends, c.rate, c.block}, limit);
+        if (p.us < 0.f) return;
+        limit = p.us;
         plan = p;
         best = ConvChoice{route, vec, vec && flat};
         d.tiles_c = (d.columns + T::BC - 1) / T::BC;
@@ -449,20 +484,39 @@ ConvChoice conv_direct_best(DirectConv &d, int batches, int kh, bool wv, bool fl
     return best;
 }
 
-// The direct kernel's plan for this convolution, or the gather core when the
-// shape is not one it takes: more than 36 taps, a transposed layer whose kernel is not its
-// stride (or padded, or cropped), an image or weight tensor of 1 GiB or more,
-// or a stride so large that no patch fits.
+ConvGeom conv_geom(const bf_cuda_conv2d_desc &d) {
+    ConvGeom g{};
+    g.N = d.batches; g.Ci = d.input_channels; g.IH = d.input_height; g.IW = d.input_width;
+    g.OH = d.output_height; g.OW = d.output_width; g.KH = d.kernel_height;
+    g.KW = d.kernel_width; g.SH = d.stride_height; g.SW = d.stride_width;
+    g.PH = d.padding_height; g.PW = d.padding_width; g.transpose = d.transpose;
+    g.M = d.batches * d.output_height * d.output_width;
+    g.K = d.input_channels * d.kernel_height * d.kernel_width;
+    return g;
+}
+
+// The direct kernel's plan for this convolution, or the gather core: when that
+// is estimated to be faster (few channels on many pixels, where the direct
+// kernel fetches and stores octets of channels that are not there; many images
+// smaller than a tile), and for shapes the direct kernel does not take: more
+// than 36 taps, a transposed layer whose kernel is not its stride (or padded, or
+// cropped), an image or weight tensor of 1 GiB or more, a stride so large that
+// no patch fits, or a grid that no launch holds.
 //
-// Tiles, by least estimate (direct_estimate): 128 x 160 (eight loader waves)
-// for full grids, 64 x 128 and 32 x 64 below, 32 x 32 where the grid would
-// leave CUs idle.  Measured on MI355X against the im2col gather: 3x3 256 -> 256
-// on 6 x 32 x 88 433 -> 39 us (515 TFLOP/s), transposed 2x2 256 -> 256 on 90 x
-// 90 376 -> 37 us.  By tile: 3x3 512 -> 128 on 64 x 64 27 us with 32 x 64 tiles
-// (40 with 64 x 128, 30 with 32 x 32), 3x3 64 -> 64 on 2 x 128 x 128 12 us with
-// 64 x 128 (18 with 128 x 160, 19 with 32 x 64).
-ConvChoice conv_direct(const bf_cuda_conv2d_desc *c, const float *x, const float *w, const float *b,
-                       float *y, DirectConv &d) {
+// Tiles: 128 x 160 (eight loader waves) for full grids, 64 x 128 and 32 x 64
+// below, 32 x 32 where the grid would leave CUs idle.  Measured on MI355X against
+// the im2col gather: 3x3 256 -> 256 on 6 x 32 x 88 433 -> 39 us (515 TFLOP/s),
+// transposed 2x2 256 -> 256 on 90 x 90 376 -> 33 us.  By tile: 3x3 512 -> 128 on
+// 64 x 64 27 us with 32 x 64 tiles (40 with 64 x 128, 30 with 32 x 32), 3x3 64 ->
+// 64 on 2 x 128 x 128 12 us with 64 x 128 (18 with 128 x 160, 19 with 32 x 64).
+// At 9293 layers the choice costs 0.8 % over the fastest kernel in the mean, and
+// at 148 of them it is more than 4 % slower than the gather core, by up to 60 %
+// (5x5 2 -> 6 on 6 x 87 x 272: 29 us, 19).  By one rate and without the stores,
+// the gather core left out where the direct kernel takes the shape, it cost 5.8 %
+// and was slower than the gather core at 5.4 %: 1x1 8 -> 8 on 5 x 187 x 470 56 us
+// (now 23), 3x3 1 -> 2 on 6 x 72 x 370 26 (10).
+ConvChoice conv_direct(const bf_cuda_conv2d_desc *c, const ConvGeom &g, const float *x, const float *w,
+                       const float *b, float *y, DirectConv &d) {
     constexpr ConvChoice kNone{kConvGather, false, false};
     d.x = x; d.w = w; d.bias = b; d.y = y;
     d.Ci = c->input_channels; d.relu = c->relu;
@@ -499,7 +553,8 @@ ConvChoice conv_direct(const bf_cuda_conv2d_desc *c, const float *x, const float
     }
     const bool wv = aligned16(w) && (c->transpose ? d.columns % 4 == 0 : (long long)d.Ci * d.khw % 4 == 0);
     const bool flat = wv && one && hw % 4 == 0 && aligned16(x);
-    return conv_direct_best(d, c->batches, kh, wv, flat);
+    const float mb = (float)g.M * (float)c->output_channels * 4e-6f;
+    return conv_direct_best(d, c->batches, kh, wv, flat, mb, conv_gather_estimate(g, c->output_channels, mb));
 }
 
 void conv_direct_run(const ConvChoice &c, const DirectConv &d, int batches, hipStream_t s) {
@@ -532,19 +587,13 @@ extern "C" int bf_cuda_conv2d_f32(const bf_cuda_conv2d_desc *d, const float *inp
         return fail(error, cap, "HIP convolution reduction is too large");
     if ((d->output_channels + 15LL) / 16 > 65535)
         return fail(error, cap, "HIP convolution has too many output channels");
-    ConvGeom g{};
-    g.N = d->batches; g.Ci = d->input_channels; g.IH = d->input_height; g.IW = d->input_width;
-    g.OH = d->output_height; g.OW = d->output_width; g.KH = d->kernel_height;
-    g.KW = d->kernel_width; g.SH = d->stride_height; g.SW = d->stride_width;
-    g.PH = d->padding_height; g.PW = d->padding_width; g.transpose = d->transpose;
-    g.M = (int)(batch_rows * d->output_width);
-    g.K = (int)(channel_reduction * d->kernel_width);
+    const ConvGeom g = conv_geom(*d);
     const int Co = d->output_channels;
     const long long tiles = ((long long)g.M + 127) / 128 * ((Co + 31LL) / 32);
     if (tiles > INT_MAX) return fail(error, cap, "HIP convolution grid is too large");
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     DirectConv direct{};
-    const ConvChoice choice = conv_direct(d, input, weight, bias, output, direct);
+    const ConvChoice choice = conv_direct(d, g, input, weight, bias, output, direct);
     if (choice.route != kConvGather)
         conv_direct_run(choice, direct, d->batches, s);
     else if (Co <= 32)
@@ -587,9 +636,9 @@ extern "C" int bfhip_gemm_route(const float *x, const float *w, const float *b, 
 extern "C" int bfhip_conv_route(const bf_cuda_conv2d_desc *desc, const float *x, const float *w,
                                 const float *y, unsigned long long *threads) {
     DirectConv d{};
-    const ConvChoice c = conv_direct(desc, x, w, nullptr, const_cast<float *>(y), d);
+    const ConvChoice c = conv_direct(desc, conv_geom(*desc), x, w, nullptr, const_cast<float *>(y), d);
     constexpr int kThreads[] = {ConvBig::kThreads, ConvMid::kThreads, ConvLow::kThreads, ConvMin::kThreads};
     *threads = c.route == kConvGather ? 0ull
                                       : (unsigned long long)d.tiles_y * d.tiles_x * d.tiles_c * desc->batches * kThreads[c.route];
-    return c.route;
+    return c.route + 8 * c.vec + 16 * c.flat;
 }

@@ -129,6 +129,11 @@ CONV_CASES = {
     "k5_s2_odd": (1, 7, 175, 21, 19, 5, 5, 2, 2, 2, 2, 11, 10, 0),
     "k3_c64": (2, 64, 576, 13, 17, 3, 3, 1, 1, 1, 1, 13, 17, 0),
     "1x1": (2, 40, 40, 8, 8, 1, 1, 1, 1, 0, 0, 8, 8, 0),
+    # layers that only the gather core takes, on its 64- and 128-column tiles
+    "gather_k7": (2, 1, 49, 11, 14, 7, 7, 1, 1, 3, 3, 11, 14, 0),
+    "gather_k7_s2": (1, 3, 147, 15, 13, 7, 7, 2, 2, 3, 3, 8, 7, 0),
+    "gather_transpose_64": (2, 7, 63, 5, 6, 3, 3, 2, 2, 1, 1, 9, 11, 1),
+    "gather_transpose_128": (1, 15, 135, 5, 4, 3, 3, 2, 2, 1, 1, 9, 7, 1),
 }
 
 
@@ -144,6 +149,9 @@ def test_conv_im2col_bit_exact(device, case):
     else:    # OIHW: W[co][k] = (co == k)
         w = np.eye(k, dtype=np.float32).reshape(k, ci, kh, kw)
     d = bfhip.ConvDesc(n, ci, k, ih, iw, kh, kw, sh, sw, ph, pw, oh, ow, tr, 0)
+    if case.startswith("gather"):
+        from test_launch_limits import conv_route
+        assert conv_route(d)[0] == 4
     wt = torch.from_numpy(np.ascontiguousarray(w)).to(device)
     digits = []
     for dgt in range(3):

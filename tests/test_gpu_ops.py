@@ -278,6 +278,61 @@ def test_conv_direct_edges(device, case, special):
     _tight(got, want, case)
 
 
+# (route, fields as CONV_CASES): every kernel at odd sizes, asserted to be the
+# one that runs (ConvRoute, + 8 with float4 weights, + 16 with float4 patches):
+# the direct tiles 128 x 160 (0), 64 x 128 (1), 32 x 64 (2) and 32 x 32 (3),
+# plain and transposed, and the gather core (4) with one, two and four blocks of
+# 32 output channels per tile, by its choice (few channels), by its taps and as
+# the padded transposed layers that only it takes.
+CONV_ROUTE_CASES = [
+    (0, (4, 16, 203, 116, 36, 1, 1, 1, 1, 0, 0, 116, 36, 0, 1)),
+    (0, (3, 17, 132, 21, 194, 3, 3, 1, 1, 1, 1, 21, 194, 0, 0)),
+    (8, (4, 92, 134, 105, 26, 1, 1, 1, 1, 0, 0, 105, 26, 0, 1)),
+    (8, (2, 2, 88, 115, 149, 6, 6, 1, 1, 3, 3, 116, 150, 0, 0)),
+    (24, (2, 28, 193, 105, 80, 1, 1, 1, 1, 0, 0, 105, 80, 0, 0)),
+    (8, (2, 85, 9, 107, 157, 2, 2, 2, 2, 0, 0, 214, 314, 1, 0)),
+    (24, (2, 33, 19, 105, 180, 2, 2, 2, 2, 0, 0, 210, 360, 1, 1)),
+    (1, (2, 1, 239, 31, 73, 1, 1, 1, 1, 0, 0, 31, 73, 0, 1)),
+    (9, (2, 44, 157, 53, 125, 1, 1, 1, 1, 0, 0, 53, 125, 0, 0)),
+    (25, (2, 60, 43, 110, 120, 1, 1, 1, 1, 0, 0, 110, 120, 0, 1)),
+    (9, (3, 1, 107, 41, 31, 2, 2, 2, 2, 0, 0, 82, 62, 1, 1)),
+    (25, (3, 1, 188, 10, 68, 2, 2, 2, 2, 0, 0, 20, 136, 1, 0)),
+    (2, (2, 2, 4, 59, 95, 1, 1, 1, 1, 0, 0, 59, 95, 0, 0)),
+    (10, (3, 12, 5, 49, 157, 1, 1, 1, 1, 0, 0, 49, 157, 0, 1)),
+    (26, (2, 4, 7, 52, 85, 1, 1, 1, 1, 0, 0, 52, 85, 0, 0)),
+    (2, (3, 4, 103, 15, 55, 2, 2, 2, 2, 0, 0, 30, 110, 1, 1)),
+    (10, (2, 1, 18, 41, 35, 2, 2, 2, 2, 0, 0, 82, 70, 1, 0)),
+    (26, (3, 1, 10, 73, 20, 2, 2, 2, 2, 0, 0, 146, 40, 1, 1)),
+    (3, (1, 2, 4, 5, 7, 1, 1, 2, 2, 0, 0, 3, 4, 0, 0)),
+    (11, (3, 20, 4, 5, 5, 1, 1, 2, 2, 0, 0, 3, 3, 0, 1)),
+    (27, (2, 4, 5, 6, 10, 1, 1, 1, 1, 0, 0, 6, 10, 0, 0)),
+    (3, (1, 264, 5, 51, 4, 2, 2, 2, 2, 0, 0, 102, 8, 1, 0)),
+    (11, (2, 1, 7, 5, 5, 2, 2, 2, 2, 0, 0, 10, 10, 1, 1)),
+    (27, (1, 1, 4, 4, 6, 2, 2, 2, 2, 0, 0, 8, 12, 1, 0)),
+    (4, (2, 1, 14, 65, 183, 1, 1, 1, 1, 0, 0, 65, 183, 0, 1)),
+    (4, (2, 1, 28, 127, 89, 2, 2, 2, 2, 0, 0, 254, 178, 1, 0)),
+    (4, (1, 9, 33, 14, 13, 7, 7, 1, 1, 3, 3, 14, 13, 0, 0)),
+    (4, (2, 5, 65, 19, 11, 7, 7, 2, 2, 3, 3, 10, 6, 0, 1)),
+    (4, (1, 11, 129, 12, 15, 7, 7, 1, 1, 3, 3, 12, 15, 0, 0)),
+    (4, (2, 10, 33, 6, 8, 2, 2, 2, 2, 1, 1, 10, 14, 1, 1)),
+    (4, (1, 12, 129, 5, 7, 3, 3, 2, 2, 1, 1, 9, 13, 1, 0)),
+]
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("route,fields", CONV_ROUTE_CASES)
+def test_conv_each_kernel(device, route, fields, special):
+    """As test_conv_direct_edges (sums of at most 1452 products)."""
+    import bfhip
+    from test_launch_limits import conv_route
+    print(f"[case] conv {fields} special={special}", flush=True)
+    assert conv_route(bfhip.ConvDesc(*fields))[0] == route
+    d, x, w, b, got = run_conv(device, fields, special)
+    want = convref.conv_abi(d, x, w, b, round_inputs=bf16_round)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+    _tight(got, want, fields)
+
+
 def test_conv_unaligned_operands(device):
     """Input, weights and output off the 16-byte grid (scalar fetches, and
     float stores in a transposed layer)."""

@@ -75,6 +75,7 @@ def test_gemm_choice_is_near_the_fastest(shape):
 
 
 def conv_route(d, aligned=True):
+    """(ConvRoute + 8 if weights go as float4 + 16 if the patch does, threads)."""
     f = bfhip.hip_lib().bfhip_conv_route
     f.argtypes = [C.c_void_p] * 4 + [C.c_void_p]
     p, threads = 4096 if aligned else 4100, C.c_ulonglong()
@@ -126,3 +127,32 @@ def test_conv_planning_is_cheap():
         return best / 300 * 1e6
 
     assert least(3) - least(7) < 1.2
+
+
+def conv_layer(n, ci, co, h, w, k, s, transpose=0):
+    p = 0 if transpose else k // 2
+    oh, ow = (h * s, w * s) if transpose else ((h + 2 * p - k) // s + 1, (w + 2 * p - k) // s + 1)
+    return bfhip.ConvDesc(n, ci, co, h, w, k, k, s, s, p, p, oh, ow, transpose, 0)
+
+
+# Microseconds on MI355X per kernel: the direct tiles with float4 weights (8-11),
+# with single floats (0-3), the gather core (4); HIP-graph replays.
+CONV_TIMES = {
+    (5, 4, 1, 72, 657, 1, 1): {8: 38.3, 9: 30.0, 10: 30.8, 11: 54.3, 0: 40.6, 1: 32.2, 2: 32.7, 3: 58.7, 4: 11.6},
+    (5, 8, 8, 187, 470, 1, 1): {8: 82.3, 9: 56.6, 10: 60.4, 11: 110.9, 0: 62.1, 1: 40.0, 2: 44.4, 3: 80.6, 4: 23.5},
+    (6, 1, 2, 72, 370, 3, 1): {0: 33.8, 1: 29.1, 2: 26.5, 3: 47.3, 4: 10.2},
+    (4, 1, 21, 108, 260, 5, 1): {0: 39.7, 1: 29.1, 2: 28.9, 3: 44.1, 4: 13.4},
+    (3, 1, 266, 78, 399, 5, 2): {0: 34.6, 1: 31.7, 2: 47.8, 3: 78.9, 4: 18.7},
+    (4, 8, 112, 197, 39, 3, 1): {8: 20.6, 9: 25.4, 10: 32.3, 11: 52.1, 0: 16.0, 1: 17.8, 2: 21.1, 3: 32.8, 4: 26.6},
+    (1, 8, 392, 187, 100, 3, 1): {8: 36.9, 9: 37.5, 10: 55.9, 11: 92.9, 0: 27.1, 1: 25.3, 2: 37.0, 3: 58.9, 4: 28.6},
+    (2, 88, 16, 110, 411, 1, 1): {8: 28.9, 9: 21.4, 10: 21.5, 11: 35.4, 0: 23.6, 1: 21.2, 2: 15.6, 3: 25.0, 4: 28.3},
+    (3, 411, 18, 17, 353, 3, 1): {0: 57.2, 1: 46.5, 2: 33.8, 3: 50.5, 4: 575.1},
+    (5, 8, 8, 29, 54, 3, 1): {8: 12.3, 9: 10.3, 10: 7.8, 11: 9.7, 0: 8.4, 1: 7.5, 2: 5.7, 3: 6.6, 4: 14.6},
+    (3, 56, 8, 43, 503, 2, 2, 1): {8: 21.4, 9: 16.2, 10: 12.2, 11: 17.1, 1: 19.5, 2: 12.2, 3: 17.7, 4: 151.9},
+}
+
+
+@pytest.mark.parametrize("layer", sorted(CONV_TIMES))
+def test_conv_choice_is_near_the_fastest(layer):
+    times = CONV_TIMES[layer]
+    assert times[conv_route(conv_layer(*layer))[0] % 16] <= 1.1 * min(times.values())
