@@ -48,3 +48,6 @@ extern "C" int bfhip_gemm_route(const float *x, const float *w, const float *b, 
 // threads of its launch (0 for the gather core).
 extern "C" int bfhip_conv_route(const bf_cuda_conv2d_desc *desc, const float *x, const float *w,
                                 const float *y, unsigned long long *threads);
+
+// For tests: the launches that insert a cloud of at most this many points.
+extern "C" int bfhip_voxel_insert_launches(unsigned points);

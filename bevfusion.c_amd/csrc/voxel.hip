@@ -178,9 +178,11 @@ __global__ __launch_bounds__(256) void rank_kernel(const unsigned *__restrict__ 
 // as one launch, 10 + 16 as two; at two points per voxel 4.4 against 2.3 + 4.6.
 // An eighth leaves a crowded voxel about as many points in the first launch as
 // one that it does not fill has in the second.  The contention falls with the
-// points: at kInsertWhole a sixth of it would be left to save part of, about
-// what the second launch costs.
-constexpr unsigned kInsertParts = 8, kInsertWhole = 16384;
+// points and the second launch costs 5 to 6 us; the two cross near 27 000
+// points (voxeliser as one launch and as two, us, alike for one, five and ten
+// sweeps: 17 000 points 44 and 50, 24 000 48 and 52, 28 000 51 and 50, 32 000 56
+// and 52, 50 000 76 and 53).
+constexpr unsigned kInsertParts = 8, kInsertWhole = 27648;
 
 __device__ __host__ __forceinline__ unsigned insert_split(unsigned count) {
     return count / kInsertParts + (count % kInsertParts != 0);
@@ -368,3 +370,5 @@ int bfhip::voxelize_count_device(bf_cuda_voxelizer *v, const float *points,
     if (!count_device || !points || !bound) return fail(error, cap, "invalid HIP voxelize buffers");
     return voxelize(v, points, count_device, bound, coords, means, voxel_count, stream, error, cap);
 }
+
+extern "C" int bfhip_voxel_insert_launches(unsigned points) { return points <= kInsertWhole ? 1 : 2; }

@@ -115,7 +115,7 @@ def test_voxelize_bit_exact(device, points, max_voxels):
         assert _voxel_gpu(vox, np.zeros((0, 5), np.float32), device)[2] == 0
 
 
-@pytest.mark.parametrize("points", [16384, 16385, 16391, 40001])
+@pytest.mark.parametrize("points", [16384, 16385, 16391, 27648, 27649, 27655, 40001])
 def test_voxelize_crowded(device, points):
     """Voxels of ten to thousands of points on both sides of the split into two
     insertion launches, descending through the cloud and shuffled: the kept

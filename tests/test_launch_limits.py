@@ -1,7 +1,8 @@
-"""The stateless operators' choice of kernel, asked without a GPU: a launch
-holds at most 2^32 - 1 threads along x (HIP refuses more), so no call may be
-given a kernel whose grid is larger, and every call that 128-row tiles hold
-must be given one.  Operand pointers serve for their alignment only."""
+"""The library's choices by size, asked on the CPU.  A launch holds at most
+2^32 - 1 threads along x (HIP refuses more), so no call may be given a kernel
+whose grid is larger, and every call that 128-row tiles hold must be given one;
+and a choice has to be near the fastest kernel measured.  Operand pointers
+serve for their alignment only."""
 
 import ctypes as C
 
@@ -72,6 +73,14 @@ GEMM_TIMES = {
 def test_gemm_choice_is_near_the_fastest(shape):
     times = GEMM_TIMES[shape]
     assert times[gemm_route(*shape)] <= 1.1 * min(times.values())
+
+
+def test_voxel_insertion_launches():
+    """One launch where it is faster (24 000 points 48 us, as two 52), two where
+    they are (32 000 points 52 us, as one 56)."""
+    f = bfhip.hip_lib().bfhip_voxel_insert_launches
+    f.argtypes = [C.c_uint]
+    assert [f(n) for n in (0, 1000, 17000, 24000, 32000, 100000)] == [1, 1, 1, 1, 2, 2]
 
 
 def conv_route(d, aligned=True):
