@@ -230,6 +230,25 @@ def test_lidar_pipeline_production_grid(device, lidar_path):
         net.close()
 
 
+@pytest.mark.parametrize("cloud", ["sweeps", "stress"])
+def test_lidar_wide_gathers_of_large_levels(device, lidar_path, cloud):
+    """Feature rows gathered through 64-bit addresses where workgroups write
+    their rows themselves (64 and 128 channels above 16 384 rows: ten sweeps hold
+    65 844 and 30 427) and where they take several row blocks (32 channels above
+    131 072 rows: the stress frame holds 155 985): bit-identical to 32-bit
+    offsets, which the tests around this one compare with the oracle."""
+    pts = bfw.synthetic_points(11, 100000, sweeps=10) if cloud == "sweeps" else bfw.stress_points(100000)
+    with bfhip.Voxelizer(bfhip.voxel_config(160000), 100000) as vox, bfhip.Model(lidar_path) as m:
+        net = bfhip.LidarBackbone(m, 1, 41, 1440, 1440, 160000)
+        print(f"[case] lidar wide gathers {cloud}", flush=True)
+        coords, means, count = vox.forward(_t(pts, device))
+        want = net.forward(coords, means, count).cpu().numpy()
+        net.lib.bfhip_lidar_offset_limit.argtypes = [ctypes.c_void_p, ctypes.c_uint]
+        net.lib.bfhip_lidar_offset_limit(net.handle, 0)
+        assert np.array_equal(net.forward(coords, means, count).cpu().numpy(), want)
+        net.close()
+
+
 def test_lidar_pipeline_reference_stress_frame(device, lidar_path):
     """The reference's own stress frame (tests/test_cuda_lidar.cu: 100k
     points, two per voxel, 50k voxels; level 1 holds 155 985 sites, just
