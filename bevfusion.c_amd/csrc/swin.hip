@@ -682,13 +682,14 @@ using MergeT2 = DmaTile<64, 64, 128, 2, 2, 3, true>;
 constexpr int kMergeLoaders2 = 4;
 
 // merge_gemm on the small-grid tiles where there are few rows (limits as
-// linear_f16's, 64-row tiles only while one fits each CU), else on T.  With
-// the linears' small-grid tiles the forward of 2 x 56 x 112 images (merges of
-// 196, 56 and 16 rows) went from 437 to 307 us on MI355X.
+// linear_f16's, 64-row tiles only while one fits each CU), else on T; by the
+// merge's own 2C outputs also where the probe runs it with others.  With the
+// linears' small-grid tiles the forward of 2 x 56 x 112 images (merges of 196,
+// 56 and 16 rows) went from 437 to 307 us on MI355X.
 template <int C, class T, int LW, class Epi>
 void merge_tiles(const bf16 *xh, int B, int H, int W, const bf16 *w, int N, const Epi &epi,
                  hipStream_t stream, const OutLnArgs *ln = nullptr) {
-    switch (few_tile_rows(B * ((H + 1) / 2) * ((W + 1) / 2), N, kFewLinear, 256)) {
+    switch (few_tile_rows(B * ((H + 1) / 2) * ((W + 1) / 2), 2 * C, kFewLinear, 256)) {
         case 16: return merge_gemm<C, FewTile128<16>, 4>(xh, B, H, W, w, N, epi, stream, ln);
         case 32: return merge_gemm<C, FewTile64<32>, 4>(xh, B, H, W, w, N, epi, stream, ln);
         case 64: return merge_gemm<C, MergeT2, kMergeLoaders2>(xh, B, H, W, w, N, epi, stream, ln);
@@ -953,8 +954,8 @@ extern "C" int bfhip_debug_swin_merge_gather(bf_cuda_swin *s, int stage, const v
     if (ok) {
         const EpiRowsF32 epi{out, nullptr, 4 * C, T2, 4 * C, 0};
         const bf16 *x = static_cast<const bf16 *>(xh);
-        // Same (C, tile, loader waves) per stage as merge_op; the reduction
-        // runs over 4C outputs here instead of 2C.
+        // Same (C, tile, loader waves) per stage and rows as merge_op, over 4C
+        // outputs here instead of 2C.
         if (stage == 0)
             merge_tiles<96, MergeT0, 0>(x, B, H, W, w, 4 * C, epi, st);
         else if (stage == 1)

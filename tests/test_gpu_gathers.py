@@ -139,10 +139,13 @@ def test_camera_conv_gather_bit_exact(device, tmp_models, shape, layer):
         neck.close()
 
 
-SWIN_SHAPES = {"production": (6, 256, 704), "odd": (2, 56, 112)}
+# The last three put stage 0, 1 and 2 on the 32-row tile (stage 1 of the last on
+# the 64-row one); the production and odd shapes take the tuned and the 16-row.
+SWIN_SHAPES = {"production": (6, 256, 704), "odd": (2, 56, 112), "rows_32_0": (2, 112, 336),
+               "rows_32_1": (4, 120, 340), "rows_32_2": (6, 160, 384)}
 
 
-@pytest.mark.parametrize("shape", ["production", "odd"])
+@pytest.mark.parametrize("shape", list(SWIN_SHAPES))
 @pytest.mark.parametrize("stage", [0, 1, 2])
 def test_swin_merge_gather_bit_exact(device, tmp_models, shape, stage):
     import torch
