@@ -119,8 +119,8 @@ constexpr int kLoaders = 4;
 constexpr int kFuserIn = 336, kFuserPad = 384;
 
 // One conv of the stage: the small-grid tiles where the map is small (58 x 78:
-// the forward 335 -> 213 us on MI355X), else the tuned tile T, on the wave-specialised core if it has three stages and
-// on the plain one if two.
+// the forward 335 -> 213 us on MI355X), else the tuned tile T, on the
+// wave-specialised core if it has three stages and on the plain one if two.
 template <class T, int K, class Epi>
 void bev_conv(const ConvLayer &l, const bf16 *a, int c0, const bf16 *b, int c1, const Epi &epi,
               hipStream_t s) {

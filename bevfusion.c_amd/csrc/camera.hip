@@ -78,8 +78,11 @@ constexpr int kS256Loaders = 4;
 inline bool use_s256(const ConvLayer &l) {
     return l.co == 256 && 2 * ((l.n * l.oh * l.ow + 159) / 160) >= 128;
 }
-// Between the small-grid tiles and those: 64-row tiles on the same pipeline
-// while they are at most one per CU (8192 pixels at 256 outputs).
+// Between the small-grid tiles and those (4097 to 8192 pixels at 256 outputs):
+// 64 x 128 tiles on the same pipeline, six stages, at most one per CU.  Against the
+// plain core's 64 x 128 tiles the neck takes 110 us instead of 140 on 2 x 32 x 66
+// maps, 112 instead of 142 on 2 x 32 x 88 and 113 instead of 145 on 4 x 32 x 63
+// (MI355X, graph replays); the results are the same.
 using SMid = DmaTile<64, 128, 64, 2, 2, 6, true>;
 inline bool use_smid(const ConvLayer &l) {
     return l.co == 256 && 2 * ((l.n * l.oh * l.ow + 63) / 64) <= 256;

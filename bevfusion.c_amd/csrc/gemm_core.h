@@ -796,10 +796,11 @@ inline void launch_gemm_spec(const ALoad &al, const BLoad &bl, const Epi &epi, i
 // stages in flight while most of the chip idles: the time then is the bytes
 // one workgroup reads, whatever the input's size.  There a layer runs on the
 // smallest of three tiles 64 columns wide whose grid still fits: 16, 32 or 64
-// rows on the wave-specialised core with four loader waves and as many stages
-// as the LDS holds, 128-deep k-steps where the operands allow them (half the
-// barriers; twice the bytes a loader wave keeps in flight).  `limit` bounds
-// the tiles of 16 and 32 rows, `limit64` those of 64; 0: the tuned tile.
+// rows on the wave-specialised core with four loader waves (two where a stage's
+// rows are fewer than four waves' chunks) and four to eight stages, 128-deep
+// k-steps where the operands allow them (half the barriers; twice the bytes a
+// loader wave keeps in flight).  `limit` bounds the tiles of 16 and 32 rows,
+// `limit64` those of 64; 0: the tuned tile.
 // Every tile sums k in the same order, so the choice does not change results.
 template <int ROWS>
 using FewTile128 = DmaTile<ROWS, 64, 128, ROWS == 16 ? 1 : 2, ROWS == 16 ? 4 : 2, ROWS == 64 ? 4 : 6, true>;

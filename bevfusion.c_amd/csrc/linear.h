@@ -14,9 +14,11 @@
 // stage-3 fc1; stage-1 fc1 (1584 tiles of 64 x 128) as 32-deep k-steps in
 // three stages, whose 36 KiB of LDS let four workgroups share a CU (1.55
 // rounds instead of 2.06 at three: 18.9 vs 19.7 us).  (N, K)
-// identifies the layer, so the table holds for any camera count whose grid
-// the small-grid rule below does not take (stage-2 proj is the one layer of six
-// full-size cameras that it does); other shapes take the 64-deep default.
+// identifies the layer, so the table holds for any camera count whose grid the
+// small-grid rule below does not take.  Of six full-size cameras' layers it takes
+// stage-2 proj and fc2 and stage-3 proj and fc2, the latter three on the same
+// tiles as the table (LinearSpec64, LinearSpec128); other shapes take the 64-deep
+// default.
 //
 // Four layers measured faster on the wave-specialised pipeline
 // (gemm_spec_kernel: loader waves issue every DMA, so the compute waves'
@@ -59,6 +61,10 @@ inline void linear_spec(const bf16 *x, const bf16 *w, int M, int N, int K, const
     DmaRowsBf16<T::BN, T::BK, LW * kWave> bl{w, K, N, K};
     launch_gemm_spec<T>(al, bl, epi, M, N, K, s);
 }
+
+// The 64 x 64 tiles of the wave-specialised pipeline, four loader waves each.
+using LinearSpec64 = FewTile64<64>;
+using LinearSpec128 = DmaTile<64, 64, 128, 2, 2, 3, true>;
 
 enum LinearTile { kK32, kK64, kK128, kTall, kWide, kWideXcd2, kWide32, kSpecBig, kSpec64, kSpec128 };
 
@@ -103,8 +109,8 @@ inline void linear_f16(const bf16 *x, const bf16 *w, int M, int N, int K, const 
             case 32: return linear_spec<FewTile64<32>, 4>(x, w, M, N, K, epi, s);
             case 64:
                 if (K >= 768 && (M + 63) / 64 * (N / 64) <= 256)
-                    return linear_spec<DmaTile<64, 64, 128, 2, 2, 3, true>, 4>(x, w, M, N, K, epi, s);
-                return linear_spec<FewTile64<64>, 4>(x, w, M, N, K, epi, s);
+                    return linear_spec<LinearSpec128, 4>(x, w, M, N, K, epi, s);
+                return linear_spec<LinearSpec64, 4>(x, w, M, N, K, epi, s);
             default: break;
         }
     switch (pick_linear_tile(N, K)) {
@@ -118,8 +124,8 @@ inline void linear_f16(const bf16 *x, const bf16 *w, int M, int N, int K, const 
             break;
         case kWide32: linear_tile<DmaTile<64, 128, 32, 2, 2, 3, true>>(x, w, M, N, K, epi, s); break;
         case kSpecBig: linear_spec<DmaTile<128, 128, 64, 2, 4, 2, true>, 4>(x, w, M, N, K, epi, s); break;
-        case kSpec64: linear_spec<DmaTile<64, 64, 64, 2, 2, 4, true>, 4>(x, w, M, N, K, epi, s); break;
-        case kSpec128: linear_spec<DmaTile<64, 64, 128, 2, 2, 3, true>, 4>(x, w, M, N, K, epi, s); break;
+        case kSpec64: linear_spec<LinearSpec64, 4>(x, w, M, N, K, epi, s); break;
+        case kSpec128: linear_spec<LinearSpec128, 4>(x, w, M, N, K, epi, s); break;
     }
 }
 
