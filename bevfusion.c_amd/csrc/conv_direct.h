@@ -370,13 +370,26 @@ struct DirectPlan {
     int TH, TW, O, patch_w, patch, tiles_y, tiles_x;
 };
 
+// The fewest blocks that tile T's weight slots take the reduction in.
+template <class T>
+inline float direct_blocks(const DirectConv &d) {
+    const int most = T::kSlots / d.khw;
+    return (float)(((d.Ci + 7) / 8 + most - 1) / most);
+}
+
+// A bound of tile T's estimates: no rectangle does better than whole tiles of
+// pixels, no patch and the fewest blocks.
+template <class T>
+inline float direct_bound(const DirectConv &d, int batches, const DirectCost &c) {
+    const long long grid = ((long long)d.OH * d.OW + T::BP - 1) / T::BP * ((d.columns + T::BC - 1) / T::BC) * batches;
+    return 0.999f * direct_estimate<T>(c, grid, direct_blocks<T>(d), 0.032f * (float)(T::BC * d.khw) * (float)((d.Ci + 7) / 8));
+}
+
 // Tile T's plan with the least estimate below `limit`; none when no rectangle's
 // patch fits, an offset could leave 32 bits or the grid is more than a launch
 // holds.  quads: whole quads of slots per block (WV); flat: rectangles of whole
-// pixel quads (XV).  This runs on every call, so tiles and rectangles are
-// dropped as soon as a bound of their estimate (the reduction fetched as one
-// block) reaches the limit.  Planned one after the other in full, 3x3 256 -> 256
-// on 6 x 32 x 88 took 2.6 us of host time; now 0.3 (random layers 0.9, now 0.4).
+// pixel quads (XV).  A rectangle is dropped as soon as its own bound reaches the
+// limit.
 template <class T>
 inline DirectPlan direct_plan(const DirectConv &d, int batches, int kh, bool quads, bool flat, const DirectCost &c,
                               float limit) {
@@ -384,12 +397,8 @@ inline DirectPlan direct_plan(const DirectConv &d, int batches, int kh, bool qua
     const int most = T::kSlots / d.khw < octets ? T::kSlots / d.khw : octets;  // octets per block, before rounding
     const long long wrow = d.up_h ? d.columns : d.khw, hw = (long long)d.IH * d.IW;
     const long long across = (long long)((d.columns + T::BC - 1) / T::BC) * batches;
+    const float fewest = direct_blocks<T>(d);
     DirectPlan best;
-    // No rectangle does better than whole tiles of pixels and no patch at all.
-    const float weights_kb = 0.032f * (float)(T::BC * d.khw);
-    const long long pixels = (long long)d.OH * d.OW;
-    if (0.999f * direct_estimate<T>(c, (pixels + T::BP - 1) / T::BP * across, 1.f, weights_kb * (float)octets) >= limit)
-        return best;
     constexpr int kHeights[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 32, 64};
 #pragma clang loop unroll(full)
     for (int i = 0; i < 13; ++i) {
@@ -404,7 +413,7 @@ inline DirectPlan direct_plan(const DirectConv &d, int batches, int kh, bool qua
         const int ty = (d.OH + th - 1) / th, tx = in_row > 1 ? (d.OW + tw - 1) / tw : 1, patch = (int)area;
         const long long grid = (long long)ty * tx * across;
         const float octet_kb = 0.032f * (float)(T::BC * d.khw + patch);
-        if (0.999f * direct_estimate<T>(c, grid, 1.f, octet_kb * (float)octets) >= limit) continue;
+        if (0.999f * direct_estimate<T>(c, grid, fewest, octet_kb * (float)octets) >= limit) continue;
         int o = T::kUnits / patch;  // octets per block: what fits, spread evenly over the blocks
         if (o > most) o = most;
         if (o < 1) continue;
