@@ -12,6 +12,7 @@
 #include "internal.h"
 
 #include <climits>
+#include <cstring>
 
 using namespace bfhip;
 
@@ -456,12 +457,19 @@ float conv_gather_estimate(const ConvGeom &g, int Co, float mb) {
     return c.launch + sqrtf(fetch * fetch + wait * wait) + c.store * mb;
 }
 
-// Fills in the plan with the least estimate below the gather core's, `limit`;
-// the gather core when there is none.  This runs on every call: tiles are planned
-// in the order of their bounds, and only while a bound is below the best plan
-// (host time with every tile planned in full, and so: 3x3 256 -> 256 on 6 x 32 x
-// 88 2.6 and 0.4 us; 3x3 64 -> 64 on 20 x 20 2.4 and 0.25).
-ConvChoice conv_direct_best(DirectConv &d, int batches, int kh, bool wv, bool flat, float mb, float limit) {
+// A layer's kernel and, for the direct ones, its plan.
+struct ConvPlanned {
+    ConvChoice choice;
+    DirectPlan plan;
+    int tiles_c;
+};
+
+// The plan with the least estimate below the gather core's, `limit`; the gather
+// core when there is none.  Tiles are planned in the order of their bounds, and
+// only while a bound is below the best plan (host time with every tile planned
+// in full, and so: 3x3 256 -> 256 on 6 x 32 x 88 2.6 and 0.4 us; 3x3 64 -> 64 on
+// 20 x 20 2.4 and 0.25).
+ConvPlanned conv_plan(const DirectConv &d, int batches, int kh, bool wv, bool flat, float mb, float limit) {
     struct Offer { float bound; int id; } offers[8];  // id: route + 4 vec
     int count = 0;
     const auto cost = [&](int id) {
@@ -484,8 +492,7 @@ ConvChoice conv_direct_best(DirectConv &d, int batches, int kh, bool wv, bool fl
         for (; at > 0 && offers[at - 1].bound > bound; --at) offers[at] = offers[at - 1];
         offers[at] = Offer{bound, id};
     }
-    DirectPlan plan{};
-    ConvChoice best{kConvGather, false, false};
+    ConvPlanned best{{kConvGather, false, false}, {}, 0};
     for (int i = 0; i < count && offers[i].bound < limit; ++i) {
         const int id = offers[i].id;
         const bool vec = id >= 4;
@@ -494,15 +501,34 @@ ConvChoice conv_direct_best(DirectConv &d, int batches, int kh, bool wv, bool fl
             const DirectPlan p = direct_plan<T>(d, batches, kh, vec && !d.up_h, vec && flat, cost(id), limit);
             if (p.us < 0.f) return;
             limit = p.us;
-            plan = p;
-            best = ConvChoice{(ConvRoute)(id % 4), vec, vec && flat};
-            d.tiles_c = (d.columns + T::BC - 1) / T::BC;
+            best = ConvPlanned{{(ConvRoute)(id % 4), vec, vec && flat}, p, (d.columns + T::BC - 1) / T::BC};
         });
     }
-    d.TH = plan.TH; d.TW = plan.TW; d.O = plan.O; d.patch_w = plan.patch_w; d.patch = plan.patch;
-    d.tiles_y = plan.tiles_y; d.tiles_x = plan.tiles_x;
     return best;
 }
+
+// The plans of the layers that a thread called last: a network calls the same
+// few over and over.  An entry is found by everything that a plan depends on,
+// and holds no address; a layer that is not there is planned (host time of a
+// call: 0.05 us with its plan in the table, 0.1 to 0.5 without).
+struct ConvPlanTable {
+    static constexpr unsigned kEntries = 32;
+    struct Key {
+        bf_cuda_conv2d_desc desc;
+        int loads;  // 1: float4 weights, 2: float4 patch
+    };
+    struct Entry {
+        Key key;  // zero batches: empty
+        ConvPlanned planned;
+    } entries[kEntries];
+    Entry &at(const Key &k) {
+        static_assert(sizeof(Key) == 16 * sizeof(int), "compared as words");
+        const int *w = reinterpret_cast<const int *>(&k);
+        unsigned h = 0;
+        for (int i = 0; i < 16; ++i) h = (h + (unsigned)w[i]) * 0x9e3779b1u;
+        return entries[h >> 27];
+    }
+};
 
 ConvGeom conv_geom(const bf_cuda_conv2d_desc &d) {
     ConvGeom g{};
@@ -573,8 +599,18 @@ ConvChoice conv_direct(const bf_cuda_conv2d_desc *c, const ConvGeom &g, const fl
     }
     const bool wv = aligned16(w) && (c->transpose ? d.columns % 4 == 0 : (long long)d.Ci * d.khw % 4 == 0);
     const bool flat = wv && one && hw % 4 == 0 && aligned16(x);
-    const float mb = (float)g.M * (float)c->output_channels * 4e-6f;
-    return conv_direct_best(d, c->batches, kh, wv, flat, mb, conv_gather_estimate(g, c->output_channels, mb));
+    static thread_local ConvPlanTable table;
+    const ConvPlanTable::Key key{*c, wv + 2 * flat};
+    ConvPlanTable::Entry &e = table.at(key);
+    if (std::memcmp(&e.key, &key, sizeof key) != 0) {
+        const float mb = (float)g.M * (float)c->output_channels * 4e-6f;
+        e.planned = conv_plan(d, c->batches, kh, wv, flat, mb, conv_gather_estimate(g, c->output_channels, mb));
+        e.key = key;
+    }
+    const DirectPlan &p = e.planned.plan;
+    d.TH = p.TH; d.TW = p.TW; d.O = p.O; d.patch_w = p.patch_w; d.patch = p.patch;
+    d.tiles_y = p.tiles_y; d.tiles_x = p.tiles_x; d.tiles_c = e.planned.tiles_c;
+    return e.planned.choice;
 }
 
 void conv_direct_run(const ConvChoice &c, const DirectConv &d, int batches, hipStream_t s) {

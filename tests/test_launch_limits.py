@@ -116,26 +116,50 @@ def test_conv_route_of_very_many_pixels():
 
 
 def test_conv_planning_is_cheap():
-    """The direct kernel is planned on every call.  Host time of asking for a
-    3x3 layer's plan beyond that of a layer that is not planned (49 taps), the
-    least of 30 runs; planning every tile in full took 2.6 us here."""
+    """Host time of asking for the plans of 200 different 3x3 layers (more than a
+    thread keeps) beyond that of layers that are not planned (49 taps), the least
+    of 30 runs; planning every tile in full took 2.6 us a layer here."""
     import time
     f = bfhip.hip_lib().bfhip_conv_route
     f.argtypes = [C.c_void_p] * 4 + [C.c_void_p]
     threads = C.c_ulonglong()
 
     def least(k):
-        d = bfhip.ConvDesc(6, 256, 256, 32, 88, k, k, 1, 1, k // 2, k // 2, 32, 88, 0, 0)
-        args = (C.addressof(d), 4096, 4096, 4096, C.addressof(threads))
+        layers = [bfhip.ConvDesc(6, 256, 256, h, 88, k, k, 1, 1, k // 2, k // 2, h, 88, 0, 0)
+                  for h in range(16, 216)]
+        args = [(C.addressof(d), 4096, 4096, 4096, C.addressof(threads)) for d in layers]
         best = float("inf")
         for _ in range(30):
             t = time.perf_counter()
-            for _ in range(300):
-                f(*args)
+            for a in args:
+                f(*a)
             best = min(best, time.perf_counter() - t)
-        return best / 300 * 1e6
+        return best / len(layers) * 1e6
 
     assert least(3) - least(7) < 1.2
+
+
+def test_conv_plans_kept_by_a_thread():
+    """Many layers in turn, each with and without aligned operands, get the plan
+    that a thread with nothing kept gives them."""
+    import random
+    import threading
+    rng = random.Random(7)
+    calls = []
+    for _ in range(60):
+        tr = rng.random() < 0.3
+        k = 2 if tr else rng.choice((1, 3, 5))
+        d = conv_layer(rng.randint(1, 6), rng.randint(1, 200), rng.randint(1, 200), rng.randint(5, 90),
+                       rng.randint(5, 120), k, 2 if tr else rng.choice((1, 2)), int(tr))
+        calls += [(d, True), (d, False)]
+    turn = [rng.choice(calls) for _ in range(600)]
+    got = [conv_route(*c) for c in turn]
+    fresh = {}
+    for i, c in enumerate(calls):
+        t = threading.Thread(target=lambda: fresh.__setitem__(i, conv_route(*c)))
+        t.start()
+        t.join()
+    assert got == [fresh[calls.index(c)] for c in turn]
 
 
 def conv_layer(n, ci, co, h, w, k, s, transpose=0):
