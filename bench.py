@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark: 6-camera 256x704 Swin-T + FPN + depth-head forward on one MI355X.
 
-Workload (the config the metric is quoted on):
+Workload (the one the metric is quoted on):
 images [6,3,256,704] U[0,1] ImageNet-normalised and dense depth [6,1,256,704]
 |N(0,1)|, 20 distinct frames (seeds 0-19) resident in HBM; random-init
 weights ~N(0,0.02) under the checkpoint's tensor names (no network for the
@@ -42,7 +42,7 @@ ROOT = pathlib.Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT / "bevfusion.c_amd"))
 
 # Algorithmic work per frame (6 cameras): GEMM flops 2*M*N*K with window rows
-# including padding tokens; see DESIGN.md "Measurement".
+# including padding tokens.
 GFLOP_FRAME = 304.4
 PEAK_BF16_TFLOPS = 2500.0
 PEAK_HBM_GBS = 8000.0
@@ -612,7 +612,7 @@ def downsample_leg(neck, dev, stream, reps, kernels):
             "layers": layers}
 
 
-# one fp32 linear as in Swin-T stage-1 QKV, X[11264 x 96]
+# One fp32 linear as in Swin-T stage-1 QKV, X[11264 x 96]
 # W[288 x 96] + bias, N(0,1)/sqrt(96), seed 0 (reference CPU kernels_ref.c:
 # 292-339 and its dispatch test tests/test_cpu_dispatch.c:25-70; GPU entry
 # point bf_cuda_gemm_f32, src/cuda_ops.cu:188-208).
@@ -1390,7 +1390,7 @@ def main():
         return
     if args.gpus != 1:
         print(json.dumps({"error": "this build runs on one GPU only; the path shards per camera "
-                                   "across GPUs by design (DESIGN.md) but no multi-GPU run is "
+                                   "across GPUs by design but no multi-GPU run is "
                                    "part of it", "n_gpus": args.gpus}))
         sys.exit(2)
     import numpy as np

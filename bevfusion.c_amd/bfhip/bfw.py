@@ -146,8 +146,8 @@ def relative_position_index(window: int = 7) -> np.ndarray:
 class _Init:
     """Weight initialisation policy.
 
-    ``mode="baseline"``: every weight ~N(0, 0.02), as BASELINE.json configs
-    2-4 state.  ``mode="fan_in"``: weights ~N(0, gain/sqrt(fan_in)) so every
+    ``mode="baseline"``: every weight ~N(0, 0.02), as the image
+    workloads are stated.  ``mode="fan_in"``: weights ~N(0, gain/sqrt(fan_in)) so every
     residual branch contributes O(1) to its output; the parity tests use it
     so that a wrong branch cannot hide under the residual stream.
     """
@@ -463,7 +463,7 @@ def synthetic_bev(seed: int, height=180, width=180, batches=1) -> np.ndarray:
 
 
 # --------------------------------------------------------------------------
-# Synthetic frame inputs
+# Synthetic frame inputs (six 256 x 704 cameras)
 # --------------------------------------------------------------------------
 IMAGENET_MEAN = np.array([0.485, 0.456, 0.406], dtype=np.float32)
 IMAGENET_STD = np.array([0.229, 0.224, 0.225], dtype=np.float32)

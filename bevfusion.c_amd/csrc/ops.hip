@@ -29,7 +29,7 @@ void gemm_f32_launch(const float *x, const float *w, const float *b, float *y, i
     launch_gemm<T>(al, bl, epi, M, N, K, s);
 }
 
-// Short reductions (K <= 128, the stateless linear of BASELINE config 1):
+// Short reductions (K <= 128, the linear 11264 x 96 -> 288):
 // one pass per row panel with every load issued up front, instead of the
 // tiled core's K/32 rounds of global -> registers -> LDS -> MFMA.  The grid
 // is (row panels of 128) x (2 column halves).  A workgroup copies its half
@@ -43,8 +43,8 @@ void gemm_f32_launch(const float *x, const float *w, const float *b, float *y, i
 // tiled core rounds them, the k order of the accumulation is the same
 // (32-deep MFMA steps in increasing k) and the bias is added after it, so the
 // two paths agree bit for bit.  Requires K % 4 == 0, N % 4 == 0 and 16-byte
-// aligned X, W, bias and Y.  Measured on MI355X at config 1 (M = 11264,
-// K = 96, N = 288; HIP-graph replays): 8.05 us (the tiled core: 8.8 us).
+// aligned X, W, bias and Y.  Measured on MI355X at M = 11264, K = 96,
+// N = 288 (HIP-graph replays): 8.05 us (the tiled core: 8.8 us).
 // Staging W per workgroup is what costs: with all 288 columns in one
 // workgroup and W converted through registers it took 6.3 of 12.5 us; half
 // the columns per workgroup and eight waves brought that form to 7.8 us,

@@ -144,7 +144,7 @@ def test_synthetic_checkpoint_is_deterministic():
     assert a["vtransform.depthnet.6.weight"].shape == (198, 256, 1, 1)
     assert a["neck.lateral_convs.1.conv.weight"].shape == (256, 1152, 1, 1)
     w = a["image_backbone.stages.0.blocks.0.attn.w_msa.qkv.weight"]
-    assert abs(w.std() - 0.02) < 0.002  # BASELINE.json init N(0, 0.02)
+    assert abs(w.std() - 0.02) < 0.002  # init N(0, 0.02)
 
 
 def test_rng_is_standard_normal():

@@ -2,7 +2,7 @@
 
 Follows the reference's tests/test_cuda_bev_stage.cu: the three outputs of
 one forward against the oracle stage (:58-69), a repeat (:75), and the
-production 180x180 shape (:94-118).  Tolerance: the north-star bar for
+production 180x180 shape (:94-118).  Tolerance: the bar for
 bf16-operand / fp32-accumulate outputs (rel-L2 <= 1e-2, max-abs <= 5e-2 RMS,
 tests/util.py).  Weights are fan-in initialised (gain 1.4) so every layer's
 output stays O(1) through the 18 convolutions.

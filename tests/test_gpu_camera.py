@@ -131,7 +131,7 @@ def test_neck_forward_equals_fpn_then_depth(device, tmp_models):
 
 
 def test_neck_production_batch_invariance_and_repeat(device, tmp_models):
-    """6x32x88 production neck (BASELINE config 4's camera shape; reference
+    """6x32x88 production neck (reference
     gate tests/test_cuda_camera_full.cu:69-72 repeats the production chain and
     compares bit for bit): repeated forwards are bit-identical, camera k of
     the 6-camera forward is bit-identical to the 1-camera forward of the same

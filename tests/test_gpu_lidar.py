@@ -9,7 +9,7 @@ synthetic frame.  Bars:
     order; "later point wins" is an order-free integer max);
   * voxeliser: coordinates, voxel count and MeanVFE means bit-exact, in the
     CPU's first-encounter voxel order, through both caps;
-  * sparse encoder: the dense BEV within the north-star tolerance (rel-L2
+  * sparse encoder: the dense BEV within the tolerance of tests/util.py (rel-L2
     <= 1e-2, max-abs <= 5e-2 RMS) -- its GEMMs take split fp16 operands
     (hi + lo) with fp32 accumulation -- and zero at every cell where the
     oracle's BEV has no site;

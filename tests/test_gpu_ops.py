@@ -3,11 +3,11 @@
 Cases follow the reference's own GPU operator test (tests/test_cuda_ops.cu):
 the 19x23->17 ReLU GEMM, a strided conv, a 5x5/s4 conv with Inf/NaN injected,
 a 2x2/s2 transposed conv and a 1 048 561-row grid (65 536 row tiles), all with
-its pattern() fill, plus BASELINE.json config 1 (11264x96 -> 288).
+its pattern() fill, plus the stage-1 QKV linear 11264x96 -> 288.
 
 Two references per case:
   * the fp32 CPU oracle / float64 restatement of the operator, held to the
-    north-star bf16 tolerance (tests/util.py);
+    bf16 tolerance of tests/util.py;
   * the same float64 sum over bf16-rounded operands, held to 1e-5 relative:
     it isolates the kernel's indexing from bf16 input rounding, so a wrong
     tap, row or channel cannot hide inside the bf16 tolerance.
@@ -125,7 +125,7 @@ def test_gemm_reference_fixture(device):
 
 
 def test_gemm_config1_matches_oracle(device):
-    """BASELINE.json config 1: X[11264x96] W[288x96] + bias, ~N(0,1)/sqrt(96), seed 0."""
+    """X[11264x96] W[288x96] + bias, ~N(0,1)/sqrt(96), seed 0."""
     import oracle
     import bfhip
     from bfhip import bfw

@@ -69,7 +69,7 @@ def test_swin_tiles_agree_across_batches(device, tmp_models, shape):
 
 
 def test_swin_baseline_init_matches_oracle(device, tmp_models):
-    """BASELINE.json weight init (N(0,0.02)) at one production camera."""
+    """Weights ~N(0,0.02) at one production camera."""
     from bfhip import bfw
     path = tmp_models("baseline", 0)
     images = bfw.synthetic_images(0, 1, 256, 704)

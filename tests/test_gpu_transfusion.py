@@ -7,7 +7,7 @@ one forward against the CPU decoder, a repeat, and the decoded detections.
 Bars: proposal labels, indices and the NMS'd query scores bit-exact (the
 scores are the reference's two-branch logistic with a correctly rounded exp,
 so the selection is the same total order); every floating-point field within
-the north-star tolerance (rel-L2 <= 1e-2, max-abs <= 5e-2 RMS, tests/util.py)
+the tolerance rel-L2 <= 1e-2, max-abs <= 5e-2 RMS (tests/util.py)
 -- the key side and the cross attention run fp16 operands with fp32
 accumulation.  Shapes cover a single cell, every candidate selected
 (zero-score ties), key counts that are not a multiple of the 64-key step, and

@@ -2,7 +2,7 @@
 
 import numpy as np
 
-# Tolerance stated by BASELINE.json north_star for bf16-in / fp32-accumulate
+# Tolerance of bf16-in / fp32-accumulate
 # floating-point outputs against the fp32 CPU oracle.
 REL_L2 = 1e-2
 MAX_ABS_RMS = 5e-2
