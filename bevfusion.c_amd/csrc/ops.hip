@@ -280,12 +280,6 @@ struct GemmCost {
     GemmRoute route;
     int rows, cols, depth, per_cu, threads;  // the workgroup's tile and its k-block
     float launch, each, rate, block, store, flow;
-    float us(long long grid, float blocks, float kb, float mb) const {
-        const float alone = (float)((grid + 255) / 256) * (kb / rate + each), all = (float)grid * kb / (256.f * flow);
-        const float fetch = alone > all ? alone : all;
-        const float wait = (float)((grid + 256 * per_cu - 1) / (256 * per_cu)) * blocks * block;
-        return launch + sqrtf(fetch * fetch + wait * wait) + store * mb;
-    }
 };
 // Fitted on MI355X to the times of every kernel at 3989 shapes (rows to
 // 400 000, K and N to 8192, most of them spread over the logarithm of sizes up
@@ -327,9 +321,17 @@ GemmRoute gemm_route(int M, int K, int N, bool panel) {
     const float mb = (float)M * (float)N * 4e-6f;
     float best = INFINITY;
     GemmRoute pick = kGemmNone;
+    // Every call pays for this (35 ns): a kernel whose launch, stores and longer
+    // part alone are above the best one needs no square root.
     const auto offer = [&](const GemmCost &c, long long grid, float blocks, float kb) {
-        const float us = c.us(grid, blocks, kb, mb);
-        if (us < best && launch_fits(grid, c.threads)) {
+        const float rest = best - (c.launch + c.store * mb);
+        const float alone = (float)((grid + 255) / 256) * (kb * (1.f / c.rate) + c.each);
+        const float all = (float)grid * kb * (1.f / (256.f * c.flow));
+        const float fetch = alone > all ? alone : all;
+        const float wait = (float)((grid + 256 * c.per_cu - 1) / (256 * c.per_cu)) * blocks * c.block;
+        if (fetch >= rest || wait >= rest || !launch_fits(grid, c.threads)) return;
+        const float us = c.launch + c.store * mb + sqrtf(fetch * fetch + wait * wait);
+        if (us < best) {
             best = us;
             pick = c.route;
         }
